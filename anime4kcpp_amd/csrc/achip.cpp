@@ -296,33 +296,29 @@ hipError_t launch_pass(const ACHipNet* net, int precision, int config, int stype
         return launch_mfma32(config, stype, dtype, src, sstride, w, h, dst, dstride, net->wts, net->wa32, stream);
     if (precision == ACHIP_FP32)
         return launch_fp32(config - kMfma32ConfigCount, stype, dtype, src, sstride, w, h, dst, dstride, net->wts, stream);
-    return launch_mfma(precision == ACHIP_BF16, config, stype, dtype, src, sstride, w, h, dst, dstride, net->wts,
-                       precision == ACHIP_BF16 ? net->wabf16 : net->wa16, net->wa32, stream);
+    return launch_stream16(precision == ACHIP_BF16, config, stype, dtype, src, sstride, w, h, dst, dstride, net->wts,
+                           precision == ACHIP_BF16 ? net->wabf16 : net->wa16, net->wa32, compute_units(net->device), stream);
 }
 
 hipError_t launch_batch(const ACHipNet* net, int precision, int config, int stype, int dtype, const BatchDesc* desc,
-                        int n, int total, int* counter, int max_wg, hipStream_t stream)
+                        int n, int total, int tile_rows, int* counter, int max_wg, hipStream_t stream)
 {
     if (precision == ACHIP_FP32 && config < kMfma32ConfigCount)
         return launch_mfma32_batch(config, stype, dtype, desc, n, total, counter, net->wts, net->wa32, max_wg, stream);
     if (precision == ACHIP_FP32)
         return launch_fp32_batch(config - kMfma32ConfigCount, stype, dtype, desc, n, total, counter, net->wts, max_wg,
                                  stream);
-    return launch_mfma_batch(precision == ACHIP_BF16, config, stype, dtype, desc, n, total, counter, net->wts,
-                             precision == ACHIP_BF16 ? net->wabf16 : net->wa16, net->wa32, max_wg, stream);
+    return launch_stream16_batch(precision == ACHIP_BF16, stype, dtype, desc, n, total, tile_rows, counter, net->wts,
+                                 precision == ACHIP_BF16 ? net->wabf16 : net->wa16, net->wa32, max_wg, stream);
 }
 
-// Without a tuned entry: config 0, except that the 16-bit forms take their 64x64 tile at 1024
-// threads (config 1) for inputs wider than u8.  Config 0's 64x32 tile at 512 threads wins by
-// running two workgroups per CU, and only with u8 input do two fit the CU's 160 KB of LDS
-// (80 KB each; 85 KB with 16-bit input, 95 KB with f32).  Measured: 4K f32 -> 8K -> 16K in FP16
-// took 1.55 ms with config 0 against 1.28 ms with config 1.
+// Without a tuned entry: config 0.
 int auto_config(const ACHipNet* net, int precision, int stype, int dtype, int w, int h)
 {
     std::lock_guard<std::mutex> lk(g_tune_mtx);
     auto it = g_tune.find(tune_key(net->device, precision, stype, dtype, w, h));
     if (it != g_tune.end()) return it->second;
-    return precision != ACHIP_FP32 && stype != U8 ? 1 : 0;
+    return 0;
 }
 
 int record_error(int code, const char* msg)
@@ -355,7 +351,7 @@ static int check_disjoint_writes(BatchSpan* spans, int count)
 }
 
 int batch_prepare(ACHipNet* net, int precision, int config, int src_type, int dst_type, const ACHipImage* images, int n,
-                  const void* workspace, size_t ws_bytes, char* host, BatchSpan* spans, int* total_tiles)
+                  const void* workspace, size_t ws_bytes, char* host, BatchSpan* spans, int* total_tiles, int* tile_rows)
 {
     if (precision != ACHIP_FP32 && precision != ACHIP_FP16 && precision != ACHIP_BF16)
         return fail(ACHIP_EINVAL, "precision %d not available", precision);
@@ -383,9 +379,12 @@ int batch_prepare(ACHipNet* net, int precision, int config, int src_type, int ds
         const uintptr_t s0 = reinterpret_cast<uintptr_t>(im.src), d0 = reinterpret_cast<uintptr_t>(im.dst);
         spans[ns++] = { s0, s0 + static_cast<size_t>(im.h - 1) * im.src_stride + static_cast<size_t>(im.w) * (src_type & 0xff), false, i };
         spans[ns++] = { d0, d0 + static_cast<size_t>(2 * im.h - 1) * im.dst_stride + static_cast<size_t>(2 * im.w) * (dst_type & 0xff), true, i };
-        const int tx = (im.w + tw - 1) / tw, ty = (im.h + th - 1) / th;
-        desc[i] = BatchDesc{ im.src, im.dst, im.src_stride, im.dst_stride, im.w, im.h, tx, static_cast<int>(total), 0 };
-        total += static_cast<long>(tx) * ty;
+        desc[i] = BatchDesc{ im.src, im.dst, im.src_stride, im.dst_stride, im.w, im.h, (im.w + tw - 1) / tw, 0, 0 };
+    }
+    if (precision != ACHIP_FP32) th = stream16_batch_rows(config, desc, n, compute_units(net->device));
+    for (int i = 0; i < n; i++) {
+        desc[i].first_tile = static_cast<int>(total);
+        total += static_cast<long>(desc[i].tiles_x) * ((desc[i].h + th - 1) / th);
         if (total > (1L << 30)) return fail(ACHIP_EINVAL, "batch too large (%ld tiles)", total);
     }
     // Every launch writes the workspace and each dst while it reads each src: no written span
@@ -394,11 +393,12 @@ int batch_prepare(ACHipNet* net, int precision, int config, int src_type, int ds
     const int r = check_disjoint_writes(spans, ns);
     if (r) return r;
     *total_tiles = static_cast<int>(total);
+    *tile_rows = th;
     return ACHIP_OK;
 }
 
-int batch_launch(ACHipNet* net, int precision, int config, int src_type, int dst_type, int n, int total, void* workspace,
-                 const char* host, hipStream_t st)
+int batch_launch(ACHipNet* net, int precision, int config, int src_type, int dst_type, int n, int total, int tile_rows,
+                 void* workspace, const char* host, hipStream_t st)
 {
     DeviceGuard g(net->device);
     if (g.err != hipSuccess) return hip_fail(g.err, "hipSetDevice");
@@ -407,7 +407,8 @@ int batch_launch(ACHipNet* net, int precision, int config, int src_type, int dst
     hipError_t e = hipMemcpyAsync(workspace, host, achip_batch_workspace_bytes(n), hipMemcpyHostToDevice, st);
     if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(batch descriptors)");
     auto* ddesc = reinterpret_cast<const BatchDesc*>(static_cast<char*>(workspace) + kBatchHeaderBytes);
-    e = launch_batch(net, precision, config, src_type, dst_type, ddesc, n, total, static_cast<int*>(workspace), 0, st);
+    e = launch_batch(net, precision, config, src_type, dst_type, ddesc, n, total, tile_rows,
+                     static_cast<int*>(workspace), 0, st);
     if (e != hipSuccess) return hip_fail(e, "batch kernel launch");
     return ACHIP_OK;
 }
@@ -824,7 +825,7 @@ int achip_config_count(int precision)
     switch (precision) {
     case ACHIP_FP32: return achip::kMfma32ConfigCount + achip::kFp32ConfigCount;   // FP32 MFMA, then VALU
     case ACHIP_FP16:
-    case ACHIP_BF16: return achip::kMfmaConfigCount;
+    case ACHIP_BF16: return achip::kStreamConfigCount;
     default: return 0;
     }
 }
@@ -832,7 +833,7 @@ int achip_config_count(int precision)
 int achip_config_info(int precision, int i, int* tw, int* th, int* nt, int* p, int* lds_bytes)
 {
     if (i < 0 || i >= achip_config_count(precision)) return fail(ACHIP_EINVAL, "no config %d for precision %d", i, precision);
-    const achip::Fp32Config& c = precision != ACHIP_FP32        ? achip::kMfmaConfigs[i]
+    const achip::Fp32Config& c = precision != ACHIP_FP32        ? achip::kStreamConfigs[i]
                                : i < achip::kMfma32ConfigCount ? achip::kMfma32Configs[i]
                                                                : achip::kFp32Configs[i - achip::kMfma32ConfigCount];
     if (tw) *tw = c.tw;
@@ -1078,11 +1079,11 @@ int achip_pass_batch(ACHipNet* net, int precision, int config, int src_type, int
     }
     std::vector<char> host(achip_batch_workspace_bytes(n));
     std::vector<achip::BatchSpan> spans(2 * static_cast<size_t>(n) + 1);
-    int total = 0;
+    int total = 0, rows = 0;
     const int r = achip::batch_prepare(net, precision, config, src_type, dst_type, images, n, workspace, workspace_bytes,
-                                       host.data(), spans.data(), &total);
+                                       host.data(), spans.data(), &total, &rows);
     if (r) return r;
-    return achip::batch_launch(net, precision, config, src_type, dst_type, n, total, workspace, host.data(),
+    return achip::batch_launch(net, precision, config, src_type, dst_type, n, total, rows, workspace, host.data(),
                                static_cast<hipStream_t>(stream));
 }
 

@@ -39,10 +39,11 @@ namespace achip {
 hipError_t launch_pass(const ACHipNet* net, int precision, int config, int stype, int dtype, const void* src,
                        long sstride, int w, int h, void* dst, long dstride, hipStream_t stream);
 
-// One persistent batched pass over `total` tiles described by n device descriptors;
-// counter (device int) must be zero when the kernel starts.  max_wg > 0 caps the grid.
+// One persistent batched pass over `total` tiles of tile_rows rows described by n device
+// descriptors; counter (device int) must be zero when the kernel starts.  max_wg > 0 caps the
+// grid.  (The FP32 configurations have one tile height each, the 16-bit ones take any even one.)
 hipError_t launch_batch(const ACHipNet* net, int precision, int config, int stype, int dtype, const BatchDesc* desc,
-                        int n, int total, int* counter, int max_wg, hipStream_t stream);
+                        int n, int total, int tile_rows, int* counter, int max_wg, hipStream_t stream);
 
 // The configuration ACHIP_AUTO resolves to for this shape (autotuner cache, else 0).
 int auto_config(const ACHipNet* net, int precision, int stype, int dtype, int w, int h);
@@ -60,14 +61,15 @@ struct BatchSpan {
 
 // Checks a batch (achip_pass_batch's arguments; the workspace only for size, alignment and
 // overlap) and writes its header (counter 0) and descriptors into host[0 ..
-// achip_batch_workspace_bytes(n)); spans has room for 2n + 1 entries.  No allocation on the
+// achip_batch_workspace_bytes(n)); spans has room for 2n + 1 entries; *total_tiles tiles of
+// *tile_rows rows.  No allocation on the
 // success path.  Returns ACHIP_OK or an ACHIP_* code (recorded for achip_last_error).
 int batch_prepare(ACHipNet* net, int precision, int config, int src_type, int dst_type, const ACHipImage* images, int n,
-                  const void* workspace, size_t ws_bytes, char* host, BatchSpan* spans, int* total_tiles);
+                  const void* workspace, size_t ws_bytes, char* host, BatchSpan* spans, int* total_tiles, int* tile_rows);
 
 // The host-to-device copy of a prepared batch into `workspace` and the persistent launch, on
 // `stream`, with the net's device current.
-int batch_launch(ACHipNet* net, int precision, int config, int src_type, int dst_type, int n, int total, void* workspace,
+int batch_launch(ACHipNet* net, int precision, int config, int src_type, int dst_type, int n, int total, int tile_rows, void* workspace,
                  const char* host, hipStream_t stream);
 
 // Records msg for achip_last_error; returns code.

@@ -81,10 +81,10 @@ int achip_pass_batch_noalloc(ACHipNet* net, int precision, int config, int src_t
     if (r) return r;
     alignas(16) char host[kScratchBytes];
     achip::BatchSpan spans[2 * ACHIP_NOALLOC_MAX_IMAGES + 1];
-    int total = 0;
-    r = achip::batch_prepare(net, precision, config, src_type, dst_type, images, n, ws, kScratchBytes, host, spans, &total);
+    int total = 0, rows = 0;
+    r = achip::batch_prepare(net, precision, config, src_type, dst_type, images, n, ws, kScratchBytes, host, spans, &total, &rows);
     if (r) return r;
-    return achip::batch_launch(net, precision, config, src_type, dst_type, n, total, ws, host,
+    return achip::batch_launch(net, precision, config, src_type, dst_type, n, total, rows, ws, host,
                                static_cast<hipStream_t>(stream));
 }
 

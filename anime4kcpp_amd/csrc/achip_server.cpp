@@ -560,10 +560,10 @@ bool ACHipServer::build_step()
     hipError_t e = achip::launch_copy_rows(ws_host_dev[step_next], static_cast<long>(bytes), ws, static_cast<long>(bytes),
                                            static_cast<long>(bytes), 1, batch);
     if (e == hipSuccess && n)
-        e = achip::launch_batch(net, cfg.precision, config, kU8, kU8, ddesc, n, static_cast<int>(total), reinterpret_cast<int*>(ws),
+        e = achip::launch_batch(net, cfg.precision, config, kU8, kU8, ddesc, n, static_cast<int>(total), th, reinterpret_cast<int*>(ws),
                                 cfg.max_workgroups, batch);
     if (e == hipSuccess && n16)
-        e = achip::launch_batch(net, cfg.precision, config, kU16, kU16, ddesc + n, n16, static_cast<int>(total16),
+        e = achip::launch_batch(net, cfg.precision, config, kU16, kU16, ddesc + n, n16, static_cast<int>(total16), th,
                                 reinterpret_cast<int*>(ws + 64), cfg.max_workgroups, batch);
     for (const std::shared_ptr<Req>& q : finishing) {
         if (e != hipSuccess) break;
@@ -788,7 +788,7 @@ int achip_server_create(ACHipNet* net, const ACHipServerConfig* config, ACHipSer
     const bool layered = net->blocks || net->lfamily;
     if (net->lfamily && c.precision != ACHIP_FP32) return ACHIP_EINVAL;   // ArtCNN and FSRCNNX run in FP32 only
     if (c.hbm_budget == 0) c.hbm_budget = static_cast<size_t>(16) << 30;
-    if (c.step_tiles <= 0) c.step_tiles = c.precision == ACHIP_FP32 ? 2048 : 12288;   // 4.2 / 25.2 Mpix
+    if (c.step_tiles <= 0) c.step_tiles = c.precision == ACHIP_FP32 ? 2048 : 6144;   // 4.2 / 25.2 Mpix
     if (c.max_workgroups < 0) return ACHIP_EINVAL;
     auto s = std::make_unique<ACHipServer>();
     s->net = net;

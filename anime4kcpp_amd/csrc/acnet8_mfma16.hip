@@ -10,7 +10,7 @@
 //          layer in one conv16_pair, or alone before it (conv16_layer) when the pairs use all
 //   final  conv3x3 8 -> 4, pixel shuffle 2x, + the source pixel, all in FP32 from the FP32
 //          accumulators, then fromFloat to the output type
-// The MFMA work item is the ACNetLegacy 16-bit kernel's (acnet_mfma.hip): 16 consecutive pixels
+// The MFMA work item is the ACNetLegacy 16-bit kernel's (acnet_stream16.hpp): 16 consecutive pixels
 // x 2 output rows from a 4 x 3 input patch, K = 96 over three MFMAs (one per patch column),
 // lane group g = lane/16 holding patch row g, so each lane's B operand is the 8 channels of one
 // pixel (one 16-byte LDS read); lane l's D registers are 4 channels (4 (g & 1) ..) of pixel

@@ -116,6 +116,22 @@ __device__ inline void store_pair(T* p, float a, float b)
     }
 }
 
+// the same with the caller's knowledge of the pair's alignment
+template <typename T>
+__device__ inline void store_pair_as(T* p, float a, float b, bool paired)
+{
+    using One = typename Bits<T>::one;
+    using Two = typename Bits<T>::two;
+    const T va = from_float<T>(a), vb = from_float<T>(b);
+    if (paired) {
+        *reinterpret_cast<Two*>(p) = static_cast<Two>(__builtin_bit_cast(One, va)) |
+                                     (static_cast<Two>(__builtin_bit_cast(One, vb)) << (8 * sizeof(T)));
+    } else {
+        p[0] = va;
+        p[1] = vb;
+    }
+}
+
 __device__ inline int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
 } // namespace achip

@@ -74,13 +74,17 @@ extern const int kFp32ConfigCount;
 hipError_t launch_fp32(int cfg, int stype, int dtype, const void* src, long sstride, int W, int H,
                        void* dst, long dstride, const float* wts, hipStream_t stream);
 
-// Fused pass with layers 1..8 on 16-bit MFMA and layer 0 on FP32 MFMA.  bf16 = 0: FP16
-// operands, 1: BF16 operands; wa is the per-lane A-operand blob of that type, wa0 the
-// FP32 blob's layer-0 part (acnet_device.hpp layouts).
-extern const Fp32Config kMfmaConfigs[];
-extern const int kMfmaConfigCount;
-hipError_t launch_mfma(int bf16, int cfg, int stype, int dtype, const void* src, long sstride, int W, int H,
-                       void* dst, long dstride, const float* wts, const void* wa, const float* wa0, hipStream_t stream);
+// Pass with layers 1..8 on 16-bit MFMA and layer 0 on FP32 MFMA, streamed row by row through
+// all layers (acnet_stream16.hpp).  bf16 = 0: FP16 operands, 1: BF16 operands; wa is the
+// per-lane A-operand blob of that type, wa0 the FP32 blob's layer-0 part (acnet_device.hpp
+// layouts); cus the device's compute units.
+extern const Fp32Config kStreamConfigs[];
+extern const int kStreamConfigCount;
+hipError_t launch_stream16(int bf16, int cfg, int stype, int dtype, const void* src, long sstride, int W, int H,
+                           void* dst, long dstride, const float* wts, const void* wa, const float* wa0, int cus,
+                           hipStream_t stream);
+// Rows per tile of a batch of n images (their sizes) under configuration cfg.
+int stream16_batch_rows(int cfg, const BatchDesc* desc, int n, int cus);
 
 // Fused pass with every conv layer on FP32 MFMA (tile 64 x 32; configuration 0: 1024
 // threads, 1: 512); wa32 is the per-lane FP32 A-operand blob (acnet_device.hpp layout).
@@ -225,8 +229,8 @@ hipError_t launch_copy_runs(const void* src, long ss, int spx, int soff, void* d
 // Persistent batched launches: `counter` (device int, zero at launch) is the tile queue.
 hipError_t launch_fp32_batch(int cfg, int stype, int dtype, const BatchDesc* desc, int n, int total, int* counter,
                              const float* wts, int max_wg, hipStream_t stream);
-hipError_t launch_mfma_batch(int bf16, int cfg, int stype, int dtype, const BatchDesc* desc, int n, int total,
-                             int* counter, const float* wts, const void* wa, const float* wa0, int max_wg,
-                             hipStream_t stream);
+hipError_t launch_stream16_batch(int bf16, int stype, int dtype, const BatchDesc* desc, int n, int total, int rows,
+                                 int* counter, const float* wts, const void* wa, const float* wa0, int max_wg,
+                                 hipStream_t stream);
 
 } // namespace achip

@@ -3,7 +3,7 @@
 // bias, ReLU and the deconv run in FP32 on the vector units.  Features stay f32 in LDS,
 // so the result stays within the FP32 tolerance of the reference CPU path.
 //
-// Same work item as the 16-bit MFMA kernel (acnet_mfma.hip): 16 consecutive pixels x 2
+// Same work item as the 16-bit MFMA kernel (acnet_stream16.hpp): 16 consecutive pixels x 2
 // output rows from a 4 x 3 input patch, D[16 x 16] = A[16 x 96] B[96 x 16], all 16 MFMA
 // rows useful (8 channels x 2 rows).  With K = 4 per instruction, lane group g = lane/16
 // holds patch row g and one MFMA covers one (patch column t, channel c): 24 MFMAs per
@@ -91,7 +91,14 @@ struct FlatRegion {
     }
 };
 
-// Replicate ring and zeroed border tiles: see fill_ring in acnet_mfma.hip.
+// Replicate ring.  After a layer of margin m has written its in-image region, copy the
+// image's edge pixels one pixel outward wherever the margin-m band reaches past the image
+// border.  The next layer then reads every tap without clamping and still sees the
+// reference's per-layer replicate border (Common.hpp:122-143).  Interior tiles need none.
+// (A row pair whose second row lies outside a cut region still reads input row y+2 for
+// it, with zero weights for row y -- but 0 x NaN is NaN.  In a tile whose band touches the
+// image border such a row may never be written, so those tiles zero the plane first;
+// interior tiles only read unwritten pixels for columns whose results are discarded.)
 template <int TW, int TH, int NT, int ES>
 __device__ inline void fill_ring32(float4* __restrict__ pa, float4* __restrict__ pb, int x0, int y0, int W, int H, int m)
 {

@@ -1,0 +1,70 @@
+"""The streamed 16-bit ACNetLegacy pass (stream16.hpp): strips of 64 output columns, any even
+number of rows per strip.  Sizes at the edges of strips (one column more and less than 64 and
+128, images narrower than a strip's margin, odd heights, one row more and less than the
+128-row strips of configuration 1) against the FP64 restatement with test_gpu_mfma's bounds;
+the two configurations cut the image differently and must agree bit for bit, as must a batch
+and the same images alone."""
+import numpy as np
+import pytest
+import torch
+
+from anime4kcpp_amd import hip, synth
+from oracle_lib import oracle_pass_f64, to_float
+from test_gpu_mfma import BOUNDS, err_report
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 1), (2, 1), (1, 5), (7, 9), (8, 16), (9, 2), (63, 127), (64, 128), (65, 129), (71, 31), (72, 33), (73, 3),
+         (127, 130), (129, 257), (136, 40), (200, 1), (1, 140)]
+
+
+@pytest.fixture(scope="module")
+def net(cuda):
+    n = hip.Net("hdn2", 0)
+    yield n
+    n.close()
+
+
+@pytest.mark.parametrize("prec", ["fp16", "bf16"])
+@pytest.mark.parametrize("w,h", SIZES)
+def test_strip_edges(net, weights, cuda, prec, w, h):
+    src = synth.flat_shaded(800 + w + 3 * h, w, h)
+    s = torch.from_numpy(src).to(cuda)
+    got = net.upscale(s, precision=prec, config=0)
+    other = net.upscale(s, precision=prec, config=1)
+    torch.cuda.synchronize()
+    assert torch.equal(got, other)
+    k, b = weights["hdn2"]
+    mx, mean, _ = err_report(got.cpu().numpy(), oracle_pass_f64(to_float(src), k, b))
+    assert mx <= BOUNDS[prec][0] and mean <= BOUNDS[prec][1]
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16, np.float16, np.float32])
+def test_types_and_strides(net, cuda, dtype):
+    """Every element type, from views with a pitch of their own (odd element offsets, so output
+    pairs that no single store can take), equals the packed image's result."""
+    w, h = 131, 77
+    host = synth.flat_shaded(5, w, h, dtype=np.float32)
+    top = {np.uint8: 255, np.uint16: 65535}.get(dtype)
+    arr = (host * top + 0.5).astype(dtype) if top else host.astype(dtype)
+    s = torch.from_numpy(arr).to(cuda)
+    want = net.upscale(s, precision="fp16")
+    big = torch.zeros((h, w + 5), dtype=s.dtype, device=cuda)
+    big[:, 3:3 + w] = s
+    out = torch.zeros((2 * h, 2 * w + 7), dtype=s.dtype, device=cuda)
+    net.upscale(big[:, 3:3 + w], out[:, 1:1 + 2 * w], precision="fp16")
+    torch.cuda.synchronize()
+    assert torch.equal(out[:, 1:1 + 2 * w], want)
+    around = out.cpu().numpy()
+    assert not around[:, 0].any() and not around[:, 1 + 2 * w:].any()
+
+
+@pytest.mark.parametrize("prec", ["fp16", "bf16"])
+@pytest.mark.parametrize("config", [0, 1])
+def test_batch_of_edges(net, cuda, prec, config):
+    srcs = [torch.from_numpy(synth.flat_shaded(900 + i, w, h, dtype=np.uint8)).to(cuda) for i, (w, h) in enumerate(SIZES)]
+    out = net.upscale_batch(srcs, precision=prec, config=config)
+    for i, s in enumerate(srcs):
+        alone = net.upscale(s, precision=prec)
+        torch.cuda.synchronize()
+        assert torch.equal(out[i], alone), SIZES[i]
