@@ -19,7 +19,29 @@
 #include "acnet_device.hpp"
 #include "acnet_kernels.hpp"
 
+namespace achip {
+
+int compute_units(int device)
+{
+    static std::mutex mtx;
+    static std::map<int, int> cache;
+    std::lock_guard<std::mutex> lk(mtx);
+    auto it = cache.find(device);
+    if (it != cache.end()) return it->second;
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) {
+        (void)hipGetLastError();
+        n = 256;
+    }
+    cache[device] = n;
+    return n;
+}
+
+} // namespace achip
+
 namespace {
+
+using achip::compute_units;
 
 thread_local std::string g_error;
 
@@ -227,22 +249,6 @@ std::tuple<int, int, int, int, int, int> tune_key(int device, int precision, int
 
 // the autotuner's form for achip_pass_ws, same key: true = the layer-split form
 std::map<std::tuple<int, int, int, int, int, int>, bool> g_split;
-
-int compute_units(int device)
-{
-    static std::mutex mtx;
-    static std::map<int, int> cache;
-    std::lock_guard<std::mutex> lk(mtx);
-    auto it = cache.find(device);
-    if (it != cache.end()) return it->second;
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) {
-        (void)hipGetLastError();
-        n = 256;
-    }
-    cache[device] = n;
-    return n;
-}
 
 // The form achip_pass_ws runs: the layer-split one only for FP32 ACNetLegacy passes, and there
 // the autotuner's verdict for the size class, else the rule measured on MI355X (u8 1080p:
@@ -760,7 +766,7 @@ int achip_pass8_precision(ACHipNet* net, int precision, const void* src, long sr
                                    net->a8wa, workspace, st)
             : achip::launch_acnet8_16(precision == ACHIP_BF16, net->blocks, src_type, dst_type, src, src_stride, w, h, dst,
                                       dst_stride, net->a8wts, precision == ACHIP_BF16 ? net->a8wabf16 : net->a8wa16,
-                                      workspace, st);
+                                      workspace, compute_units(net->device), st);
     return e == hipSuccess ? ACHIP_OK : hip_fail(e, "kernel launch");
 }
 

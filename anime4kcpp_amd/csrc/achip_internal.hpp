@@ -72,6 +72,9 @@ int batch_prepare(ACHipNet* net, int precision, int config, int src_type, int ds
 int batch_launch(ACHipNet* net, int precision, int config, int src_type, int dst_type, int n, int total, int tile_rows, void* workspace,
                  const char* host, hipStream_t stream);
 
+// Compute units of a device (256 where the runtime does not say).
+int compute_units(int device);
+
 // Records msg for achip_last_error; returns code.
 int record_error(int code, const char* msg);
 

@@ -296,7 +296,8 @@ hipError_t ACHipServer::pass_launch(int pcfg, int T, const Plane& a, const Plane
 {
     if (net->blocks && cfg.precision != ACHIP_FP32)
         return achip::launch_acnet8_16(cfg.precision == ACHIP_BF16, net->blocks, T, T, a.ptr, a.stride, a.w, a.h, b.ptr, b.stride,
-                                       net->a8wts, cfg.precision == ACHIP_BF16 ? net->a8wabf16 : net->a8wa16, ws.ptr, st);
+                                       net->a8wts, cfg.precision == ACHIP_BF16 ? net->a8wabf16 : net->a8wa16, ws.ptr,
+                                       achip::compute_units(net->device), st);
     if (net->blocks)
         return achip::launch_acnet8(net->blocks, T, T, a.ptr, a.stride, a.w, a.h, b.ptr, b.stride, net->a8wts, net->a8wa, ws.ptr, st);
     if (net->lfamily == kNetArtCNN)

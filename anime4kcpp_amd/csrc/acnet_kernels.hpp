@@ -112,13 +112,14 @@ hipError_t launch_legacy_split(int stype, int dtype, const void* src, long ss, i
 hipError_t launch_legacy_split_batch(int stype, int dtype, const SplitDesc* desc, int n, int total, const float* wts,
                                      const float* wa32, hipStream_t stream);
 
-// ACNet<8> 2x pass with the conv3x3 layers on 16-bit MFMA (acnet8_mfma16.hip): bf16 = 0 FP16,
-// 1 BF16 operands; wa16 that type's per-lane A operands of the blocks and the final layer
-// (3 x 64 x 8 values per layer, final layer rows 4-7 zero).  Workspace: two 16-bit maps of
-// acnet8_map16_pitch(W) * H bytes (fits in the FP32 path's workspace).
+// ACNet<8> 2x pass with the conv3x3 layers on 16-bit MFMA, streamed (acnet8_stream16.hpp):
+// bf16 = 0 FP16, 1 BF16 operands; wa16 that type's per-lane A operands of the blocks and the
+// final layer (3 x 64 x 8 values per layer, final layer rows 4-7 zero); cus the device's
+// compute units.  Workspace: two 16-bit maps of acnet8_map16_pitch(W) * H bytes (fits in the
+// FP32 path's workspace); nets of up to 8 blocks do not touch it.
 long acnet8_map16_pitch(int w);
 hipError_t launch_acnet8_16(int bf16, int blocks, int stype, int dtype, const void* src, long ss, int W, int H, void* dst,
-                            long ds, const float* wts, const void* wa16, void* workspace, hipStream_t stream);
+                            long ds, const float* wts, const void* wa16, void* workspace, int cus, hipStream_t stream);
 
 // ArtCNN<F> 2x pass, F = 16 or 32 (artcnn.hip): kernels/biases in the reference layout
 // (device copies), wa the per-lane A operands of the B body layers, the residual layer and

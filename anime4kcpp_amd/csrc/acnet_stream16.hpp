@@ -174,7 +174,7 @@ __device__ __forceinline__ void legacy_strip(const void* __restrict__ src, long 
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const StripRows sr(y0, y1, H, kSLLayers);
+    const StripRows sr(y0, y1, H, kSLLayers, 1);
     const int nsteps = sr.steps(), xs = x0 - kSLMargin;
     const bool edge = xs < 0 || xs + kSCols > W;
     char* const ring0 = lds + 16;
@@ -195,7 +195,7 @@ __device__ __forceinline__ void legacy_strip(const void* __restrict__ src, long 
         if (edge) legacy_first<T16, 0, 3, true>(W, xs, sr, nsteps, wts, wa0, img, ring0, lane);
         else legacy_first<T16, 0, 3, false>(W, xs, sr, nsteps, wts, wa0, img, ring0, lane);
     } else if (wave == kSLWaves - 1) {
-        strip_loader<TIN>(src, ss, W, H, xs, sr, nsteps, img, lane);
+        image_loader<TIN>(src, ss, W, H, xs, sr, nsteps, img, lane);
     } else {
         const int l = wave < 8 ? 2 * (wave - 4) + 1 : 2 * (wave - 8) + 2;
         const LegacyOp<T16> op(l, wts, wa, lane);
@@ -259,7 +259,7 @@ static hipError_t launch_one(int cfg, const void* src, long ss, int W, int H, vo
                              const uint4* wa, const float* wa0, int cus, hipStream_t stream)
 {
     const int strips = (W + kSLOut - 1) / kSLOut;
-    const int rows = cfg ? kStreamConfigs[cfg].th : strip_rows(strips, H, kSLLayers, cus);
+    const int rows = cfg ? kStreamConfigs[cfg].th : strip_rows(strips, H, kSLLayers, cus, 2);
     hipLaunchKernelGGL((acnet_stream16<T16, TIN, TOUT>), dim3(strips, (H + rows - 1) / rows), dim3(kSLThreads), 0, stream,
                        src, ss, W, H, dst, ds, wts, wa, wa0, rows);
     return hipGetLastError();

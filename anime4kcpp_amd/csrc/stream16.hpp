@@ -58,14 +58,18 @@ struct RingRow {
 // The rows and steps of the layers 0 .. last of a strip with output rows [y0, y1) (y1 - y0
 // even, or y1 the image's end).  Layer l's pair p is rows base(l) + 2p, + 1; pairs that lie
 // outside the image are left out.
+// lead: 1 where a loader fills layer 0's source rows (it counts as layer -1), 0 where the loader
+// fills layer 0's ring itself.
 struct StripRows {
     int y0, y1, H, last, s0;
-    __device__ __forceinline__ StripRows(int y0_, int y1_, int H_, int last_) : y0(y0_), y1(y1_), H(H_), last(last_), s0(0) { s0 = first(0); }
+    __device__ __forceinline__ StripRows(int y0_, int y1_, int H_, int last_, int lead) : y0(y0_), y1(y1_), H(H_), last(last_), s0(0)
+    {
+        s0 = first(0) - kSLag * lead;
+    }
     __device__ __forceinline__ int base(int l) const { return y0 - (last - l); }
     __device__ __forceinline__ int first(int l) const { return max(-base(l), 0) >> 1; }
     __device__ __forceinline__ int end(int l) const { return (min(y1 + (last - l), H) - base(l) + 1) >> 1; }
-    // the loader's rows count as layer -1, whose first pair is step 0
-    __device__ __forceinline__ int step(int l, int p) const { return p + kSLag * (l + 1) - s0; }
+    __device__ __forceinline__ int step(int l, int p) const { return p + kSLag * l - s0; }
     __device__ __forceinline__ int steps() const { return step(last, end(last)); }
     // Whether pair p's patch reaches outside the image, and for those pairs the offset of patch
     // row g in the ring of layer l - 1: the nearest row inside.
@@ -76,9 +80,61 @@ struct StripRows {
     }
 };
 
-// ---- the loader: source rows as f32 in a ring of three pairs ----
-// Image columns xs - 1 .. xs + 80 and rows base(0) - 1 .., clamped to the image, converted once
-// (layer 0's items read each pixel up to 12 times).
+// ---- loaders ----
+// One wave: pairs first .. end - 1 of rows row0 + 2p, + 1 (clamped to the image) of the columns
+// xs .. xs + COLS - 1 (clamped) into a ring, put(row of the pair, column, element) storing one
+// element and next() moving on by a pair.  The rows of the next AHEAD pairs are in flight in
+// registers: a step is shorter than a load's latency.
+template <typename T, int COLS, int AHEAD, class Put, class Next>
+__device__ __forceinline__ void strip_loader(const void* __restrict__ src, long ss, int W, int H, int xs, int row0, int first,
+                                             int end, int nsteps, int lane, Put put, Next next)
+{
+    static_assert(COLS > 64 && COLS <= 96, "three elements per lane and pair");
+    // lane: column lane of both rows, and column 64 + lane % 32 of row lane / 32
+    const int ct = 64 + (lane & 31);
+    const int c0 = clampi(xs + lane, 0, W - 1), c2 = clampi(xs + ct, 0, W - 1);
+    const bool low = lane < 32, tail = ct < COLS;
+    int row = row0 + 2 * first;
+    T v[AHEAD][3];
+    auto fetch = [&](T (&t)[3]) {
+        const T* r0 = row_ptr<T>(src, ss, clampi(row, 0, H - 1));
+        const T* r1 = row_ptr<T>(src, ss, clampi(row + 1, 0, H - 1));
+        t[0] = r0[c0];
+        t[1] = r1[c0];
+        t[2] = (low ? r0 : r1)[c2];
+        row += 2;
+    };
+    auto store = [&](const T (&t)[3]) {
+        put(0, lane, t[0]);
+        put(1, lane, t[1]);
+        if (tail) put(low ? 0 : 1, ct, t[2]);
+        next();
+    };
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++) fetch(v[u]);
+    int s = 0;
+    for (int left = end - first; left >= AHEAD; left -= AHEAD) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            store(v[u]);
+            fetch(v[u]);
+            step_barrier();
+        }
+        s += AHEAD;
+    }
+    const int rest = (end - first) % AHEAD;
+#pragma unroll
+    for (int u = 0; u < AHEAD - 1; u++) {
+        if (u < rest) {
+            store(v[u]);
+            step_barrier();
+        }
+    }
+    for (s += rest; s < nsteps; s++) step_barrier();
+}
+
+// Source rows as f32 in a ring of three pairs: image columns xs - 1 .. xs + 80 and rows
+// base(0) - 1 .., converted once (layer 0's items read each pixel up to 12 times).
 constexpr int kSImgCols = kSCols + 2;
 constexpr unsigned kSImgRowBytes = (kSImgCols + 2) * 4;
 constexpr unsigned kSImgBytes = kSRows * kSImgRowBytes;
@@ -93,57 +149,15 @@ struct ImgRow {
     }
 };
 
-// One wave.  The rows of the next kSAhead pairs are in flight in registers: a step is shorter
-// than a load's latency.
-constexpr int kSAhead = 6;
 template <typename TIN>
-__device__ __forceinline__ void strip_loader(const void* __restrict__ src, long ss, int W, int H, int xs, const StripRows& sr,
+__device__ __forceinline__ void image_loader(const void* __restrict__ src, long ss, int W, int H, int xs, const StripRows& sr,
                                              int nsteps, char* img, int lane)
 {
-    // lane: column lane of both rows, and column 64 + lane % 32 of row lane / 32
-    const int c0 = clampi(xs - 1 + lane, 0, W - 1), c2 = clampi(xs - 1 + 64 + (lane & 31), 0, W - 1);
-    const bool low = lane < 32, tail = (lane & 31) < kSImgCols - 64;
-    const int first = sr.s0, end = sr.end(0) + 1;
-    int row = sr.base(0) - 1 + 2 * first;
-    TIN v[kSAhead][3];
-    auto fetch = [&](TIN (&t)[3]) {
-        const TIN* r0 = row_ptr<TIN>(src, ss, clampi(row, 0, H - 1));
-        const TIN* r1 = row_ptr<TIN>(src, ss, clampi(row + 1, 0, H - 1));
-        t[0] = r0[c0];
-        t[1] = r1[c0];
-        t[2] = (low ? r0 : r1)[c2];
-        row += 2;
-    };
-#pragma unroll
-    for (int u = 0; u < kSAhead; u++) fetch(v[u]);
-    ImgRow out(2 * first);
-    int s = 0;
-    for (int left = end - first; left >= kSAhead; left -= kSAhead) {
-#pragma unroll
-        for (int u = 0; u < kSAhead; u++) {
-            float* w = reinterpret_cast<float*>(img + out.off);
-            w[lane] = to_float<TIN>(v[u][0]);
-            w[kSImgRowBytes / 4 + lane] = to_float<TIN>(v[u][1]);
-            if (tail) w[(low ? 0 : kSImgRowBytes / 4) + 64 + (lane & 31)] = to_float<TIN>(v[u][2]);
-            fetch(v[u]);
-            out.next_pair();
-            step_barrier();
-        }
-        s += kSAhead;
-    }
-    const int rest = (end - first) % kSAhead;
-#pragma unroll
-    for (int u = 0; u < kSAhead - 1; u++) {
-        if (u < rest) {
-            float* w = reinterpret_cast<float*>(img + out.off);
-            w[lane] = to_float<TIN>(v[u][0]);
-            w[kSImgRowBytes / 4 + lane] = to_float<TIN>(v[u][1]);
-            if (tail) w[(low ? 0 : kSImgRowBytes / 4) + 64 + (lane & 31)] = to_float<TIN>(v[u][2]);
-            out.next_pair();
-            step_barrier();
-        }
-    }
-    for (s += rest; s < nsteps; s++) step_barrier();
+    ImgRow out(2 * sr.first(0));
+    strip_loader<TIN, kSImgCols, 6>(
+        src, ss, W, H, xs - 1, sr.base(0) - 1, sr.first(0), sr.end(0) + 1, nsteps, lane,
+        [&](int r, int c, TIN v) { reinterpret_cast<float*>(img + out.off + r * kSImgRowBytes)[c] = to_float<TIN>(v); },
+        [&]() { out.next_pair(); });
 }
 
 // Write items O0 .. O0 + N - 1 of a unit (res[o]: 4 channels of column O0 + o + 5 j, image
@@ -208,8 +222,13 @@ __device__ __forceinline__ void strip_layer(const Op& op, int l, int W, int xs, 
     for (; s < nsteps; s++) step_barrier();
 }
 
-// The other half's share of two sums: lane ^ 16 holds the other four channels of this lane's
-// pixel and row.  half = 0 lanes get (a of both), half = 1 lanes (b of both).
+// The two halves (lanes 16 apart) of a pixel: half = 0 lanes hold channels 0-3, half = 1 lanes
+// 4-7.  other_half: a for half = 0 lanes, the partner's b for half = 1 lanes.  add_halves: the sum
+// of both halves' a for half = 0 lanes, of both halves' b for half = 1 lanes.
+__device__ __forceinline__ float other_half(float a, float b)
+{
+    return __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false)[0]);
+}
 __device__ __forceinline__ float add_halves(float a, float b)
 {
     const auto e = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
@@ -221,28 +240,28 @@ __device__ __forceinline__ float add_halves(float a, float b)
 __device__ __forceinline__ float relu1(float v) { return __builtin_amdgcn_fmed3f(v, 0.f, __builtin_inff()); }
 
 // ---- the heights of strips (host) ----
-// Steps of a strip of `rows` output rows and `layers` layers after layer 0: its row pairs, the
-// lag of the layers and the loader, half of it again for the margins.
+// Steps of a strip of `rows` output rows and `layers` layers after layer 0: its row pairs and
+// the lag of the layers and the loader.
 inline int strip_steps(int rows, int layers) { return (rows + 1) / 2 + kSLag * (layers + 1); }
 
-// Rows per strip of an image of `strips` strips x H rows on a device of `cus` compute units.
-// Measured on 1080p and 4K u8 in FP16 (8 layers): a step takes about 0.72 us with one
-// workgroup per CU and 0.97 us with two, so the candidates are the heights that fill one
-// workgroup per CU or 1, 2, 4 rounds of two, and the cheapest by that count is taken.  1080p:
-// 64 rows 46 us (32: 56, 136: 62); 4K: 270 rows 150 (128: 149, 64: 163); 256 x 256: 4 rows
-// 12.4 (2: 14.5, 16: 17).
-inline int strip_rows(long strips, int H, int layers, int cus)
+// Rows per strip of an image of `strips` strips x H rows on a device of `cus` compute units that
+// hold per_cu workgroups each.  Measured on 1080p and 4K u8 in FP16 (8 layers, two per CU): a
+// step takes about 0.72 us with one workgroup per CU and 0.97 us with two, so the candidates are
+// the heights that fill one workgroup per CU or 1, 2, 4 rounds of all, and the cheapest by
+// that count is taken.  1080p: 64 rows 46 us (32: 56, 136: 62); 4K: 270 rows 150 (128: 149, 64:
+// 163); 256 x 256: 4 rows 12.4 (2: 14.5, 16: 17).
+inline int strip_rows(long strips, int H, int layers, int cus, int per_cu)
 {
     long best = -1;
     int rows = (H + 1) / 2 * 2;
     const int rounds[] = { 0, 1, 2, 4 };
+    const long all = static_cast<long>(per_cu) * cus;
     for (int k : rounds) {
-        const long slots = k ? 2L * cus : cus;
-        const long segs = slots * (k ? k : 1) / strips;
+        const long segs = (k ? k * all : cus) / strips;
         if (segs < 1) continue;
         const int r = static_cast<int>(((H + segs - 1) / segs + 1) / 2 * 2);
         const long n = strips * ((H + r - 1) / r);
-        const long cost = strip_steps(r, layers) * (n <= cus ? 3L : 4L * ((n + 2L * cus - 1) / (2L * cus)));
+        const long cost = strip_steps(r, layers) * (n <= cus ? 3L : (2L + per_cu) * ((n + all - 1) / all));
         if (best < 0 || cost < best) {
             best = cost;
             rows = r;

@@ -1,4 +1,4 @@
-"""The streamed 16-bit ACNetLegacy pass (stream16.hpp): strips of 64 output columns, any even
+"""The streamed 16-bit passes: ACNetLegacy (stream16.hpp): strips of 64 output columns, any even
 number of rows per strip.  Sizes at the edges of strips (one column more and less than 64 and
 128, images narrower than a strip's margin, odd heights, one row more and less than the
 128-row strips of configuration 1) against the FP64 restatement with test_gpu_mfma's bounds;
@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from anime4kcpp_amd import hip, synth
-from oracle_lib import oracle_pass_f64, to_float
+from oracle_lib import oracle_pass8_f64, oracle_pass_f64, to_float
 from test_gpu_mfma import BOUNDS, err_report
 
 pytestmark = pytest.mark.gpu
@@ -68,3 +68,40 @@ def test_batch_of_edges(net, cuda, prec, config):
         alone = net.upscale(s, precision=prec)
         torch.cuda.synchronize()
         assert torch.equal(out[i], alone), SIZES[i]
+
+
+SIZES8 = [(1, 1), (2, 9), (59, 5), (60, 16), (61, 17), (62, 70), (63, 71), (64, 30), (69, 2), (70, 12), (71, 13), (125, 68)]
+
+
+@pytest.mark.parametrize("prec", ["fp16", "bf16"])
+@pytest.mark.parametrize("variant", ["b4_hdn", "b8_hdn", "b18_box_hdn"])
+def test_acnet8_strip_edges(cuda, prec, variant):
+    """ACNet<8>: 70, 62 and (two launches) 62 and 60 output columns per strip."""
+    k, b, a, blocks = hip.load_weights8(variant)
+    net = hip.Net8(variant)
+    for w, h in SIZES8:
+        src = synth.flat_shaded(300 + w + 3 * h, w, h)
+        got = net.upscale(torch.from_numpy(src).to(cuda), precision=prec)
+        torch.cuda.synchronize()
+        mx, mean, _ = err_report(got.cpu().numpy(), oracle_pass8_f64(to_float(src), k, b, a, blocks))
+        assert mx <= BOUNDS[prec][0] and mean <= BOUNDS[prec][1], (w, h)
+    net.close()
+
+
+@pytest.mark.parametrize("blocks", [1, 2, 3, 8, 9, 10, 17, 18, 19, 27])
+def test_acnet8_crop(cuda, blocks):
+    """Every cut of the blocks into launches: a crop's outputs further than the receptive field
+    from its border are the whole image's, bit for bit, in strips that start elsewhere."""
+    k, b, a, _ = hip.load_weights8("b18_hdn")
+    pick = [i % 18 for i in range(blocks)]
+    kk = np.concatenate([k[:72]] + [k[72 + 576 * i:72 + 576 * (i + 1)] for i in pick] + [k[-288:]])
+    bb = np.concatenate([b[:8]] + [b[8 + 8 * i:16 + 8 * i] for i in pick] + [b[-4:]])
+    aa = np.concatenate([a[:8]] + [a[8 + 8 * i:16 + 8 * i] for i in pick])
+    net = hip.Net8("b4", weights=(kk, bb, aa, blocks))
+    src = torch.from_numpy(synth.flat_shaded(41, 230, 180, dtype=np.uint8)).to(cuda)
+    whole = net.upscale(src, precision="fp16", out_dtype=torch.float32)
+    x, y, w, h, m = 37, 23, 150, 121, blocks + 2
+    part = net.upscale(src[y:y + h, x:x + w], precision="fp16", out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert torch.equal(part[2 * m:2 * (h - m), 2 * m:2 * (w - m)], whole[2 * (y + m):2 * (y + h - m), 2 * (x + m):2 * (x + w - m)])
+    net.close()
