@@ -251,10 +251,11 @@ std::tuple<int, int, int, int, int, int> tune_key(int device, int precision, int
 std::map<std::tuple<int, int, int, int, int, int>, bool> g_split;
 
 // The form achip_pass_ws runs: the layer-split one only for FP32 ACNetLegacy passes, and there
-// the autotuner's verdict for the size class, else the rule measured on MI355X (u8 1080p:
-// fused 328 us, split 299 us; 4K: 1307 / 1042 us; 256 x 256: 82 / 52 us; 960 x 540: 84 /
-// 109 us): the fused kernel wins only where its grid of 64 x 32 tiles fits in one round of
-// the device's compute units and the image is larger than 256 x 256.
+// the autotuner's verdict for the size class, else this rule: the fused kernel, which needs no
+// workspace, where its 64 x 32 tiles make just about one full round of the compute units (within 4%
+// of the split form there), the split form elsewhere.  u8, fused / split us: 128 x 96 81 / 20,
+// 256 x 256 83 / 28, 720 x 480 84 / 61, 960 x 540 84 / 81 (one tile per compute unit), 1280 x 720
+// 165 / 118, 1920 x 1080 330 / 213, 3840 x 2160 1310 / 780.
 bool split_preferred(const ACHipNet* net, int precision, int st, int dt, int w, int h)
 {
     if (precision != ACHIP_FP32 || net->blocks || net->lfamily) return false;
@@ -263,8 +264,8 @@ bool split_preferred(const ACHipNet* net, int precision, int st, int dt, int w, 
         auto it = g_split.find(tune_key(net->device, precision, st, dt, w, h));
         if (it != g_split.end()) return it->second;
     }
-    const long tiles = static_cast<long>((w + 63) / 64) * ((h + 31) / 32);
-    return !(tiles <= compute_units(net->device) && static_cast<long>(w) * h > 256L * 256);
+    const long tiles = static_cast<long>((w + 63) / 64) * ((h + 31) / 32), cus = compute_units(net->device);
+    return tiles * 16 <= cus * 15 || tiles > cus;
 }
 
 } // namespace
@@ -471,6 +472,10 @@ int achip_net_create(int device, const float* kernels, const float* biases, ACHi
     const std::vector<uint16_t> a16 = mfma_operands(kernels, false);
     const std::vector<uint16_t> abf = mfma_operands(kernels, true);
     const std::vector<float> a32 = mfma32_operands(kernels);
+    std::vector<float> a4(achip::kRows8L0Floats + 8 * achip::kRows8Floats);
+    achip::pack_legacy_l0(kernels, a4.data());
+    for (int l = 0; l < 8; l++)
+        achip::pack_conv8_operands(kernels + 72 + 576 * l, 8, a4.data() + achip::kRows8L0Floats + l * achip::kRows8Floats);
 
     DeviceGuard g(device);
     if (g.err != hipSuccess) return hip_fail(g.err, "hipSetDevice");
@@ -478,7 +483,8 @@ int achip_net_create(int device, const float* kernels, const float* biases, ACHi
     const size_t off16 = (blob.size() * sizeof(float) + 255) / 256 * 256;
     const size_t offbf = off16 + achip::kMfmaBlobBytes;
     const size_t off32 = offbf + achip::kMfmaBlobBytes;
-    const size_t total = off32 + a32.size() * sizeof(float);
+    const size_t off4 = off32 + (a32.size() * sizeof(float) + 255) / 256 * 256;
+    const size_t total = off4 + a4.size() * sizeof(float);
     char* d = nullptr;
     hipError_t e = hipMalloc(&d, total);
     if (e != hipSuccess) return hip_fail(e, "hipMalloc(weights)");
@@ -486,11 +492,13 @@ int achip_net_create(int device, const float* kernels, const float* biases, ACHi
     if (e == hipSuccess) e = hipMemcpy(d + off16, a16.data(), achip::kMfmaBlobBytes, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d + offbf, abf.data(), achip::kMfmaBlobBytes, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d + off32, a32.data(), a32.size() * sizeof(float), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(d + off4, a4.data(), a4.size() * sizeof(float), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         (void)hipFree(d);
         return hip_fail(e, "hipMemcpy(weights)");
     }
-    *out = new ACHipNet{ device, reinterpret_cast<float*>(d), d + off16, d + offbf, reinterpret_cast<float*>(d + off32) };
+    *out = new ACHipNet{ device, reinterpret_cast<float*>(d), d + off16, d + offbf, reinterpret_cast<float*>(d + off32),
+                         reinterpret_cast<float*>(d + off4) };
     g_error.clear();
     return ACHIP_OK;
 }
@@ -532,9 +540,9 @@ int achip_net8_create(int device, int blocks, const float* kernels, const float*
             blob[achip::kA8OffLayer + 16 * (l - 1) + o] = biases[8 * l + o];
             blob[achip::kA8OffLayer + 16 * (l - 1) + 8 + o] = alphas[8 * l + o];
         }
-    std::vector<float> wa(static_cast<size_t>(blocks + 1) * achip::kMfma32LayerFloats);
+    std::vector<float> wa(static_cast<size_t>(blocks + 1) * achip::kRows8Floats);
     for (int l = 1; l <= blocks + 1; l++)
-        achip::pack_conv8_operands(kernels + 72 + 576 * (l - 1), l <= blocks ? 8 : 4, wa.data() + (l - 1) * achip::kMfma32LayerFloats);
+        achip::pack_conv8_operands(kernels + 72 + 576 * (l - 1), l <= blocks ? 8 : 4, wa.data() + (l - 1) * achip::kRows8Floats);
 
     // the same layers as 16-bit operands: FP16 for all layers, then BF16
     const size_t per16 = static_cast<size_t>(3) * 64 * 8;
@@ -718,7 +726,7 @@ int achip_pass_net(ACHipNet* net, const void* src, long src_stride, int src_type
             ? achip::launch_artcnn(net->lf, net->lblocks, src_type, dst_type, src, src_stride, w, h, dst, dst_stride, net->lk,
                                    net->lb, net->lwa, workspace, st)
             : achip::launch_fsrcnnx(net->lf, net->lblocks, src_type, dst_type, src, src_stride, w, h, dst, dst_stride,
-                                    net->lk, net->lb, net->la, net->lwa, net->lw1, workspace, st);
+                                    net->lk, net->lb, net->la, net->lwa, net->lw1, workspace, compute_units(net->device), st);
     return e == hipSuccess ? ACHIP_OK : hip_fail(e, "kernel launch");
 }
 
@@ -763,7 +771,7 @@ int achip_pass8_precision(ACHipNet* net, int precision, const void* src, long sr
     const hipError_t e =
         precision == ACHIP_FP32
             ? achip::launch_acnet8(net->blocks, src_type, dst_type, src, src_stride, w, h, dst, dst_stride, net->a8wts,
-                                   net->a8wa, workspace, st)
+                                   net->a8wa, workspace, compute_units(net->device), st)
             : achip::launch_acnet8_16(precision == ACHIP_BF16, net->blocks, src_type, dst_type, src, src_stride, w, h, dst,
                                       dst_stride, net->a8wts, precision == ACHIP_BF16 ? net->a8wabf16 : net->a8wa16,
                                       workspace, compute_units(net->device), st);
@@ -793,7 +801,8 @@ int achip_pass_layers(ACHipNet* net, const void* src, long src_stride, int src_t
     DeviceGuard g(net->device);
     if (g.err != hipSuccess) return hip_fail(g.err, "hipSetDevice");
     const hipError_t e = achip::launch_legacy_split(src_type, dst_type, src, src_stride, w, h, dst, dst_stride, net->wts,
-                                                    net->wa32, workspace, static_cast<hipStream_t>(stream));
+                                                    net->wa4, workspace, compute_units(net->device),
+                                                    static_cast<hipStream_t>(stream));
     return e == hipSuccess ? ACHIP_OK : hip_fail(e, "kernel launch");
 }
 
@@ -1147,9 +1156,13 @@ int achip_pass_batch_layers(ACHipNet* net, int src_type, int dst_type, const ACH
         const long fp = achip::acnet8_feature_pitch(im.w);
         auto* m0 = reinterpret_cast<float4*>(ws + offsets[i]);
         auto* m1 = reinterpret_cast<float4*>(ws + offsets[i] + static_cast<size_t>(fp) * im.h);
-        const int tx = (im.w + 61) / 62, ty = (im.h + 15) / 16;
-        desc[i] = achip::SplitDesc{ im.src, im.dst, m0, m1, im.src_stride, im.dst_stride, fp, im.w, im.h, tx, static_cast<int>(total) };
-        total += static_cast<long>(tx) * ty;
+        const int cols = achip::legacy_batch_cols();
+        desc[i] = achip::SplitDesc{ im.src, im.dst, m0, m1, im.src_stride, im.dst_stride, fp, im.w, im.h, (im.w + cols - 1) / cols, 0 };
+    }
+    const int rows = achip::legacy_batch_rows(desc.data(), n, compute_units(net->device));
+    for (achip::SplitDesc& d : desc) {
+        d.first_tile = static_cast<int>(total);
+        total += static_cast<long>(d.tiles_x) * ((d.h + rows - 1) / rows);
         if (total > (1L << 30)) return fail(ACHIP_EINVAL, "batch too large (%ld tiles)", total);
     }
     // the maps and descriptors are written by the launches: no image may overlap them, and no
@@ -1166,7 +1179,7 @@ int achip_pass_batch_layers(ACHipNet* net, int src_type, int dst_type, const ACH
                                   hipMemcpyHostToDevice, st);
     if (e == hipSuccess)
         e = achip::launch_legacy_split_batch(src_type, dst_type, reinterpret_cast<const achip::SplitDesc*>(workspace), n,
-                                             static_cast<int>(total), net->wts, net->wa32, st);
+                                             static_cast<int>(total), rows, net->wts, net->wa4, st);
     return e == hipSuccess ? ACHIP_OK : hip_fail(e, "kernel launch");
 }
 

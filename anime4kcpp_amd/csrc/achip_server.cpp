@@ -299,13 +299,14 @@ hipError_t ACHipServer::pass_launch(int pcfg, int T, const Plane& a, const Plane
                                        net->a8wts, cfg.precision == ACHIP_BF16 ? net->a8wabf16 : net->a8wa16, ws.ptr,
                                        achip::compute_units(net->device), st);
     if (net->blocks)
-        return achip::launch_acnet8(net->blocks, T, T, a.ptr, a.stride, a.w, a.h, b.ptr, b.stride, net->a8wts, net->a8wa, ws.ptr, st);
+        return achip::launch_acnet8(net->blocks, T, T, a.ptr, a.stride, a.w, a.h, b.ptr, b.stride, net->a8wts, net->a8wa, ws.ptr,
+                                    achip::compute_units(net->device), st);
     if (net->lfamily == kNetArtCNN)
         return achip::launch_artcnn(net->lf, net->lblocks, T, T, a.ptr, a.stride, a.w, a.h, b.ptr, b.stride, net->lk, net->lb,
                                     net->lwa, ws.ptr, st);
     if (net->lfamily == kNetFSRCNNX)
         return achip::launch_fsrcnnx(net->lf, net->lblocks, T, T, a.ptr, a.stride, a.w, a.h, b.ptr, b.stride, net->lk, net->lb,
-                                     net->la, net->lwa, net->lw1, ws.ptr, st);
+                                     net->la, net->lwa, net->lw1, ws.ptr, achip::compute_units(net->device), st);
     return achip::launch_pass(net, cfg.precision, pcfg, T, T, a.ptr, a.stride, a.w, a.h, b.ptr, b.stride, st);
 }
 

@@ -19,7 +19,7 @@ struct BatchDesc {
 };
 
 // One image of a batched layer-split pass: its images, its two 8-channel f32 maps (rows fp
-// bytes apart) and its 62 x 16-pixel tiles, numbered image by image from first_tile.
+// bytes apart) and its tiles, numbered image by image from first_tile.
 struct SplitDesc {
     const void* src;
     void* dst;
@@ -100,17 +100,20 @@ hipError_t launch_mfma32_batch(int cfg, int stype, int dtype, const BatchDesc* d
 // blocks and the final layer.  Workspace: 2 * acnet8_feature_pitch(W) * H bytes.
 long acnet8_feature_pitch(int w);
 hipError_t launch_acnet8(int blocks, int stype, int dtype, const void* src, long ss, int W, int H, void* dst, long ds,
-                         const float* wts, const float* wa, void* workspace, hipStream_t stream);
+                         const float* wts, const float* wa, void* workspace, int cus, hipStream_t stream);
 
-// ACNetLegacy's FP32 pass layer by layer (acnet8.hip): layer 0 into an f32 map, layers 1..8
-// two per launch, the last pair ending in the deconv; workspace as launch_acnet8 (two maps of
-// acnet8_feature_pitch(W) * H bytes).
+// ACNetLegacy's FP32 pass a few layers per launch (acnet8.hip), the fused kernel's bits; wa4 is the
+// blob of pack_legacy_l0 and eight layers of pack_conv8_operands; workspace as launch_acnet8
+// (two maps of acnet8_feature_pitch(W) * H bytes).
+constexpr int kRows8L0Floats = 2 * 64, kRows8Floats = 9 * 64;
 hipError_t launch_legacy_split(int stype, int dtype, const void* src, long ss, int W, int H, void* dst, long ds,
-                               const float* wts, const float* wa32, void* workspace, hipStream_t stream);
-// The same for n images (one element type pair) in four launches over the tiles of all of
-// them, `total` in all; desc is device memory.
-hipError_t launch_legacy_split_batch(int stype, int dtype, const SplitDesc* desc, int n, int total, const float* wts,
-                                     const float* wa32, hipStream_t stream);
+                               const float* wts, const float* wa4, void* workspace, int cus, hipStream_t stream);
+// The same for n images (one element type pair) in launches over the strips of all of them,
+// `total` in all, of legacy_batch_cols() columns and `rows` rows; desc is device memory.
+int legacy_batch_cols();
+int legacy_batch_rows(const SplitDesc* desc, int n, int cus);
+hipError_t launch_legacy_split_batch(int stype, int dtype, const SplitDesc* desc, int n, int total, int rows, const float* wts,
+                                     const float* wa4, hipStream_t stream);
 
 // ACNet<8> 2x pass with the conv3x3 layers on 16-bit MFMA, streamed (acnet8_stream16.hpp):
 // bf16 = 0 FP16, 1 BF16 operands; wa16 that type's per-lane A operands of the blocks and the
@@ -138,20 +141,21 @@ hipError_t launch_artcnn(int f, int blocks, int stype, int dtype, const void* sr
 long fsrcnnx_feature_pitch(int f, int w);
 hipError_t launch_fsrcnnx(int f, int blocks, int stype, int dtype, const void* src, long ss, int W, int H, void* dst,
                           long ds, const float* kernels, const float* biases, const float* alphas, const float* wa,
-                          const float* w1, void* workspace, hipStream_t stream);
+                          const float* w1, void* workspace, int cus, hipStream_t stream);
 
-// Host-side packing of the per-lane A operands the layer kernels (conv_layers.hpp) read.
-// F = 8 (2-row items), conv3x3 8 -> cout (8 or 4): [t * 8 + c][lane] for patch column t,
-// channel c; conv1x1 8 -> 8: [r][lane], block-diagonal over the item's two output rows.
+// Host-side packing of the A operands the layer kernels read.  F = 8 (conv8_rows.hpp), conv3x3
+// 8 -> cout (8 or 4) in kRows8Floats floats, ACNetLegacy's layer 0 in kRows8L0Floats, conv1x1
+// 8 -> 8 in 64: 16 operands of four output channels per register.
 // F = 16 or 32 (channel tiles), conv3x3 F -> F: [tap][lane][q * F/16 + h]; F -> 4 (the tail,
 // one output tile): [tap][lane][q];
 // conv1x1 F -> F: [4 h + r][lane][h2].  k in the reference layout k[n][tap][c].
 void pack_conv8_operands(const float* k, int cout, float* out);
+void pack_legacy_l0(const float* k, float* out);
 void pack_conv8_1x1(const float* k1, float* out);
 void pack_convf_operands(const float* k, int f, int cout, float* out);
 void pack_convf_1x1(const float* k1, int f, float* out);
-inline size_t conv_operand_floats(int f) { return f == 8 ? 24 * 64 : 9 * 64 * static_cast<size_t>(f / 4) * (f / 16); }
-inline size_t conv_1x1_floats(int f) { return f == 8 ? 4 * 64 : static_cast<size_t>(f / 4) * 64 * (f / 16); }
+inline size_t conv_operand_floats(int f) { return f == 8 ? kRows8Floats : 9 * 64 * static_cast<size_t>(f / 4) * (f / 16); }
+inline size_t conv_1x1_floats(int f) { return f == 8 ? 64 : static_cast<size_t>(f / 4) * 64 * (f / 16); }
 
 // ---- colour conversion and resize (acnet_color.hip) ----
 

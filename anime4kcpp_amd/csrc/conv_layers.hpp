@@ -1,9 +1,7 @@
-// The FP32 MFMA conv3x3 layer kernels of the layer-by-layer networks (ACNet<8>, ArtCNN<F>,
-// FSRCNNX<F>): one launch per layer (two for conv8_pair), reading an F-channel f32 map from
-// HBM (channel quads interleaved per pixel: pixel x at float4 index F/4 * x + q, rows of `fp`
-// bytes), and writing the next map or, for the last layer, the 2x output image.  The layer's epilogue is
-// chosen at compile time (LayerMode); every form keeps the reference's separately rounded
-// steps after the conv sum (Common.hpp:116-164, 227-288, 290-341):
+// The conv3x3 layers of the layer-by-layer networks (ACNet<8>, ArtCNN<F>, FSRCNNX<F>): their
+// epilogues (LayerMode), which keep the reference's separately rounded steps after the conv sum
+// (Common.hpp:116-164, 227-288, 290-341), and the 16- and 32-channel kernel.  The 8-channel layers
+// are conv8_rows.hpp's.
 //   kRelu          max(v, 0)                                        ArtCNN body
 //   kPrelu         max(v, 0) + a * min(v, 0)                        ACNet<8>, FSRCNNX body
 //   kAddFeat       v * 1 + feat                                     ArtCNN's last F -> F
@@ -13,21 +11,19 @@
 //   kShuffleSrc    the same, + the source pixel                     ACNet<8> final
 //   kReluDeconv    ReLU, then the 2x2 stride-2 deconv 8 -> 1 to 2x  ACNetLegacy's last layer
 //                  (Common.hpp:344-393), layer by layer
-// Two MFMA mappings (v_mfma_f32_16x16x4_f32):
-//   conv8_layer, conv8_pair  F = 8: the 2-row item of acnet_mfma32_item.hpp, 16 pixels x 2
-//                output rows per item, all 16 MFMA rows useful;
-//   convf_layer  F = 16 or 32: M = 16 output channels per tile (F/16 tiles), N = 16 pixels of
-//                one row, K = 9 taps x F; lane group g supplies input channels g*F/4 ..
-//                g*F/4 + F/4 - 1 from channel-quad LDS planes; NI items per wave batch share
-//                each tap's A operands.
-// In both, a lane's D registers hold 4 consecutive channels of one pixel, which is exactly
-// the B operand a conv1x1 MFMA needs (K step r of lane group g = the r-th of them), so the
-// fused conv1x1 costs F/4 x F/16 more MFMAs and no data movement.
+// convf_layer (F = 16 or 32): one launch per layer, reading an F-channel f32 map from HBM (channel
+// quads interleaved per pixel: pixel x at float4 index F/4 * x + q, rows of `fp` bytes), and
+// writing the next map or, for the last layer, the 2x output image.  v_mfma_f32_16x16x4_f32 with
+// M = 16 output channels per tile (F/16 tiles), N = 16 pixels of one row, K = 9 taps x F; lane
+// group g supplies input channels g*F/4 .. g*F/4 + F/4 - 1 from channel-quad LDS planes; NI items
+// per wave batch share each tap's A operands.  A lane's D registers hold 4 consecutive channels of
+// one pixel, which is exactly the B operand a conv1x1 MFMA needs (K step r of lane group g = the
+// r-th of them), so the fused conv1x1 costs F/4 x F/16 more MFMAs and no data movement.
 #pragma once
 
 #include "acnet_device.hpp"
 #include "acnet_kernels.hpp"
-#include "acnet_mfma32_item.hpp"
+#include "acnet_mfma32_item.hpp"   // mma32
 
 namespace achip {
 
@@ -90,283 +86,6 @@ __device__ __forceinline__ void stage_map(const float4* __restrict__ fin, long f
         }
     }
 }
-
-// ---- F = 8: the 2-row item ----
-// Tile: TW x TH output pixels, NT threads; the input region (with the one-pixel halo) staged
-// in LDS as two float4 planes (channels 0-3, 4-7) with a row pitch that is a multiple of 16
-// pixels (the 16-byte item reads run at full rate).  Items: 16-pixel segments x row pairs,
-// dealt to the waves round-robin.  Default 64 x 16, 256 threads: 46 KB, three workgroups
-// per CU.
-template <int TW_ = 64, int TH_ = 16, int NT_ = 256>
-struct Conv8Tile {
-    static constexpr int TW = TW_, TH = TH_, NT = NT_, NW = NT / 64;
-    static constexpr int PW = (TW + 2 + 15) / 16 * 16, PH = TH + 2;
-};
-
-// The epilogue of an 8-channel item: this lane's bias, slopes and conv1x1 operands (lane
-// (g, j) owns channels 4 half .. + 3 of output row ro of pixel j), and what it does with the
-// item's D registers.  `ok`: the lane's pixel (x, y) is an output of this tile.
-template <int MODE, typename TIN, typename TOUT>
-struct Epi8 {
-    static_assert(MODE == kRelu || MODE == kPrelu || MODE == kPreluConv1x1 || MODE == kShuffle || MODE == kShuffleSrc ||
-                      MODE == kReluDeconv,
-                  "8-channel epilogues");
-    static constexpr bool SHUFFLE = MODE == kShuffle || MODE == kShuffleSrc;
-    f32x4m bias, bias1 = { 0.f, 0.f, 0.f, 0.f };
-    float alpha[4] = { 0.f, 0.f, 0.f, 0.f }, alpha1[4] = { 0.f, 0.f, 0.f, 0.f }, w1[4] = { 0.f, 0.f, 0.f, 0.f };
-    float kd[4][4];   // kReluDeconv: this lane's 4 channels x 4 sub-pixels of k2
-
-    __device__ void load(const LayerArgs& la, int lane, int half)
-    {
-        if constexpr (MODE == kRelu || MODE == kReluDeconv) {
-            const float* bl = la.bias + 4 * half;
-            bias = (f32x4m){ bl[0], bl[1], bl[2], bl[3] };
-            if constexpr (MODE == kReluDeconv)
-#pragma unroll
-                for (int c = 0; c < 4; c++)
-#pragma unroll
-                    for (int q = 0; q < 4; q++) kd[c][q] = la.k2[(4 * half + c) * 4 + q];
-        } else if constexpr (SHUFFLE) {
-            bias = half ? (f32x4m){ 0.f, 0.f, 0.f, 0.f } : (f32x4m){ la.bias[0], la.bias[1], la.bias[2], la.bias[3] };
-        } else {
-            const float* bl = la.bias + 4 * half;
-            bias = (f32x4m){ bl[0], bl[1], bl[2], bl[3] };
-#pragma unroll
-            for (int r = 0; r < 4; r++) alpha[r] = la.alpha[4 * half + r];
-        }
-        if constexpr (MODE == kPreluConv1x1) {
-            const float* bl = la.b1 + 4 * half;
-            bias1 = (f32x4m){ bl[0], bl[1], bl[2], bl[3] };
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                alpha1[r] = la.alpha1[4 * half + r];
-                w1[r] = la.w1[r * 64 + lane];
-            }
-        }
-    }
-
-    // every lane of the wave calls this (the conv1x1 MFMAs and the shuffle take all lanes)
-    __device__ void apply(const f32x4m& acc, int x, int y, bool ok, int half, long fp, float4* __restrict__ fout,
-                          const LayerArgs& la) const
-    {
-        if constexpr (MODE == kRelu) {
-            if (ok) {
-                float4* px = reinterpret_cast<float4*>(reinterpret_cast<char*>(fout) + static_cast<long>(y) * fp) + 2 * x + half;
-                *px = make_float4(fmaxf(acc[0], 0.f), fmaxf(acc[1], 0.f), fmaxf(acc[2], 0.f), fmaxf(acc[3], 0.f));
-            }
-        } else if constexpr (MODE == kReluDeconv) {
-            // this lane's 4 channels' share of the 4 sub-pixels, plus the partner lane's
-            // (lane ^ 16 holds the other 4 channels of the same pixel and row); half = 0
-            // lanes write output row 2y (q = 0, 1), half = 1 lanes row 2y + 1 (q = 2, 3)
-            const float v0 = fmaxf(acc[0], 0.f), v1 = fmaxf(acc[1], 0.f), v2 = fmaxf(acc[2], 0.f), v3 = fmaxf(acc[3], 0.f);
-            float sum[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) sum[q] = fmaf(v3, kd[3][q], fmaf(v2, kd[2][q], fmaf(v1, kd[1][q], v0 * kd[0][q])));
-#pragma unroll
-            for (int q = 0; q < 4; q++) sum[q] += __shfl_xor(sum[q], 16);
-            if (ok) store_pair<TOUT>(row_ptr<TOUT>(la.dst, la.ds, 2 * y + half) + 2 * x, half ? sum[2] : sum[0], half ? sum[3] : sum[1]);
-        } else if constexpr (MODE == kPrelu) {
-            if (ok) {
-                float4* px = reinterpret_cast<float4*>(reinterpret_cast<char*>(fout) + static_cast<long>(y) * fp) + 2 * x + half;
-                *px = make_float4(prelu(acc[0], alpha[0]), prelu(acc[1], alpha[1]), prelu(acc[2], alpha[2]),
-                                  prelu(acc[3], alpha[3]));
-            }
-        } else if constexpr (MODE == kPreluConv1x1) {
-            // conv1x1 over (output row, channel): K step r of lane group g is channel
-            // 4 half + r of row ro -- this lane's own D register r
-            f32x4m d = bias1;
-#pragma unroll
-            for (int r = 0; r < 4; r++) d = mma32(w1[r], prelu(acc[r], alpha[r]), d);
-            if (ok) {
-                const long off = static_cast<long>(y) * fp;
-                const float4 f = *(reinterpret_cast<const float4*>(reinterpret_cast<const char*>(la.feat) + off) + 2 * x + half);
-                float4* px = reinterpret_cast<float4*>(reinterpret_cast<char*>(fout) + off) + 2 * x + half;
-                *px = make_float4(prelu(add_skip(d[0], f.x), alpha1[0]), prelu(add_skip(d[1], f.y), alpha1[1]),
-                                  prelu(add_skip(d[2], f.z), alpha1[2]), prelu(add_skip(d[3], f.w), alpha1[3]));
-            }
-        } else {
-            // lanes with half = 0 hold the four sub-pixels n = 0..3 (output (2x + n % 2,
-            // 2y + n / 2)); half = 1 lanes take row 2y + 1 from them
-            const float n2 = __shfl_xor(acc[2], 16), n3 = __shfl_xor(acc[3], 16);
-            if (ok) {
-                float s0 = half ? n2 : acc[0], s1 = half ? n3 : acc[1];
-                if constexpr (MODE == kShuffleSrc) {
-                    const float res = to_float<TIN>(row_ptr<TIN>(la.src, la.ss, y)[x]);
-                    s0 = add_skip(s0, res);
-                    s1 = add_skip(s1, res);
-                }
-                store_pair<TOUT>(row_ptr<TOUT>(la.dst, la.ds, 2 * y + half) + 2 * x, s0, s1);
-            }
-        }
-    }
-};
-
-template <int MODE, typename TIN, typename TOUT, class C = Conv8Tile<>>
-__global__ __launch_bounds__(C::NT) void conv8_layer(const float4* __restrict__ fin, long fp, int W, int H,
-                                                     float4* __restrict__ fout, const LayerArgs la)
-{
-    constexpr int kC8TW = C::TW, kC8TH = C::TH, kC8PW = C::PW, kC8PH = C::PH;
-    __shared__ float4 pa[kC8PW * kC8PH];
-    __shared__ float4 pb[kC8PW * kC8PH];
-    const int tiles_x = gridDim.x;
-    const int t = xcd_tile(blockIdx.y * tiles_x + blockIdx.x, tiles_x * gridDim.y);
-    const int ty = t / tiles_x, tx = t - ty * tiles_x;
-    const int x0 = tx * kC8TW, y0 = ty * kC8TH;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = lane >> 4, j = lane & 15, half = g & 1, ro = g >> 1;
-
-    // stage rows y0-1 .. y0+TH, columns x0-1 .. x0+TW (replicated at the image edges)
-    {
-        float4* const pl[2] = { pa, pb };
-        stage_map<C::NT, kC8TW + 2, kC8PH, 2, kC8PW>(fin, fp, W, H, x0 - 1, y0 - 1, pl);
-    }
-    float a[24];
-#pragma unroll
-    for (int s = 0; s < 24; s++) a[s] = la.wa[s * 64 + lane];
-    Epi8<MODE, TIN, TOUT> epi;
-    epi.load(la, lane, half);
-    __syncthreads();
-
-    const int gx1 = min(x0 + kC8TW, W), gy1 = min(y0 + kC8TH, H);
-    const int nseg = (gx1 - x0 + 15) >> 4;
-    const int nitems = nseg * ((gy1 - y0 + 1) >> 1);
-    const int lane_rd = g * kC8PW + j;
-    for (int item = wave; item < nitems; item += C::NW) {
-        const int pair = item / nseg, seg = item - pair * nseg;
-        // patch row g of output rows (y0 + 2 pair, +1) is staged row 2 pair + g; column j + t
-        const Item32 q = load_item(pa, pb, 2 * pair * kC8PW + 16 * seg + lane_rd);
-        const f32x4m acc = item24(q, a, epi.bias);
-        const int x = x0 + 16 * seg + j, y = y0 + 2 * pair + ro;
-        epi.apply(acc, x, y, x < gx1 && y < gy1, half, fp, fout, la);
-    }
-}
-
-// Two consecutive 8-channel layers in one launch: layer A (conv3x3 + PReLU or ReLU, arguments la0)
-// and layer B (conv3x3 with the MODE epilogue, arguments la), so the map between them stays
-// in LDS.  Output tile 62 x 16: layer A's region grows by one pixel per side to 64 x 18,
-// exactly 4 segments x 9 row pairs; the staged input is 66 x 20 (80-pixel pitch, 51 KB,
-// three workgroups per CU).  After layer A, tiles at the image edge overwrite A's pixels
-// outside the image with the nearest pixel inside, so layer B sees the replicate padding
-// every layer of the reference applies (Common.hpp:120-143).
-constexpr int kP8TW = 62, kP8TH = 16, kP8PW = 80, kP8PH = kP8TH + 4;
-// threads per two-layer workgroup, its waves, and layer A's items per wave
-constexpr int kP8NT = 256, kP8NW = kP8NT / 64, kP8AI = (36 + kP8NW - 1) / kP8NW;
-
-// The second layer of a two-layer launch, once layer A fills plane pixels (1..64, 1..18)
-// of pa/pb: the replicate ring, then layer B (A operands a, epilogue epi) over the 62 x 16 tile.
-template <int MODE, typename TIN, typename TOUT>
-__device__ __forceinline__ void pair8_second(float4* __restrict__ pa, float4* __restrict__ pb, int W, int H, int x0, int y0,
-                                             const float (&a)[24], const Epi8<MODE, TIN, TOUT>& epi, long fp,
-                                             float4* __restrict__ fout, const LayerArgs& la)
-{
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = lane >> 4, j = lane & 15, half = g & 1, ro = g >> 1;
-    const int lane_rd = g * kP8PW + j;
-    // replicate ring: A's pixels outside the image take the nearest pixel inside
-    if (x0 - 1 < 0 || y0 - 1 < 0 || x0 + kP8TW >= W || y0 + kP8TH >= H) {
-        for (int e = tid; e < 18 * 64; e += kP8NT) {
-            const int r = 1 + e / 64, c = 1 + (e & 63);
-            const int gy = y0 - 2 + r, gx = x0 - 2 + c;
-            if (gx >= 0 && gx < W && gy >= 0 && gy < H) continue;
-            const int s = (clampi(gy, 0, H - 1) - (y0 - 2)) * kP8PW + clampi(gx, 0, W - 1) - (x0 - 2);
-            pa[r * kP8PW + c] = pa[s];
-            pb[r * kP8PW + c] = pb[s];
-        }
-        __syncthreads();
-    }
-    // layer B over the 62 x 16 tile: 32 items dealt round-robin to the waves; patch rows 2 pair + 1 + g,
-    // columns 16 seg + j + t + 1 (columns past A's region feed only lanes past the tile)
-    const int gx1 = min(x0 + kP8TW, W), gy1 = min(y0 + kP8TH, H);
-    static_assert(32 % kP8NW == 0, "layer B's items split evenly over the waves");
-#pragma unroll
-    for (int ib = 0; ib < 32 / kP8NW; ib++) {   // unrolled: the next item's LDS reads issue early
-        const int item = wave + kP8NW * ib, pair = item >> 2, seg = item & 3;
-        const f32x4m acc = item24(load_item(pa, pb, (2 * pair + 1) * kP8PW + 16 * seg + 1 + lane_rd), a, epi.bias);
-        const int x = x0 + 16 * seg + j, y = y0 + 2 * pair + ro;
-        epi.apply(acc, x, y, x < gx1 && y < gy1, half, fp, fout, la);
-    }
-}
-
-
-// Layer A of a two-layer launch: its input at plane pixels (0..65, 0..19) of pa/pb, its
-// output written back to (1..64, 1..18) -- 36 items, round-robin over the waves; item (pair, seg) reads
-// patch rows 2 pair + g, columns 16 seg + j + t.  Takes layer A's A operands in `a` and its
-// epilogue in epa; returns with layer B's (la) in `a` and epi, loaded while the other waves
-// finish layer A.
-template <int MODE_A, int MODE, typename TIN, typename TOUT>
-__device__ __forceinline__ void pair8_first(float4* __restrict__ pa, float4* __restrict__ pb, float (&a)[24],
-                                            const Epi8<MODE_A, float, float>& epa, Epi8<MODE, TIN, TOUT>& epi,
-                                            const LayerArgs& la)
-{
-    static_assert(MODE_A == kPrelu || MODE_A == kRelu, "layer A: conv3x3 + PReLU or ReLU");
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = lane >> 4, j = lane & 15, half = g & 1, ro = g >> 1;
-    const int lane_rd = g * kP8PW + j;
-    float4 res[kP8AI];
-#pragma unroll
-    for (int ii = 0; ii < kP8AI; ii++) {
-        const int item = wave + kP8NW * ii, pair = item >> 2, seg = item & 3;
-        if (36 % kP8NW == 0 || item < 36) {   // uniform across the wave
-            const f32x4m acc = item24(load_item(pa, pb, 2 * pair * kP8PW + 16 * seg + lane_rd), a, epa.bias);
-            if constexpr (MODE_A == kPrelu)
-                res[ii] = make_float4(prelu(acc[0], epa.alpha[0]), prelu(acc[1], epa.alpha[1]), prelu(acc[2], epa.alpha[2]),
-                                      prelu(acc[3], epa.alpha[3]));
-            else
-                res[ii] = make_float4(fmaxf(acc[0], 0.f), fmaxf(acc[1], 0.f), fmaxf(acc[2], 0.f), fmaxf(acc[3], 0.f));
-        }
-    }
-#pragma unroll
-    for (int s = 0; s < 24; s++) a[s] = la.wa[s * 64 + lane];
-    epi.load(la, lane, half);
-    __syncthreads();
-    {
-        float4* const pw = half ? pb : pa;
-#pragma unroll
-        for (int ii = 0; ii < kP8AI; ii++) {
-            const int item = wave + kP8NW * ii, pair = item >> 2, seg = item & 3;
-            if (36 % kP8NW == 0 || item < 36) pw[(1 + 2 * pair + ro) * kP8PW + 1 + 16 * seg + j] = res[ii];
-        }
-    }
-    __syncthreads();
-}
-
-// Both layers of a two-layer launch on the tile whose output starts at (x0, y0); pa/pb are the
-// workgroup's LDS planes.
-template <int MODE, typename TIN, typename TOUT, int MODE_A>
-__device__ __forceinline__ void pair8_tile(const float4* __restrict__ fin, long fp, int W, int H, float4* __restrict__ fout,
-                                           const LayerArgs& la0, const LayerArgs& la, int x0, int y0,
-                                           float4* __restrict__ pa, float4* __restrict__ pb)
-{
-    const int lane = threadIdx.x & 63, half = (lane >> 4) & 1;
-    // plane pixel (c, r) is image pixel (x0 - 2 + c, y0 - 2 + r); stage 66 x 20, clamped
-    {
-        float4* const pl[2] = { pa, pb };
-        stage_map<kP8NT, kP8TW + 4, kP8PH, 2, kP8PW>(fin, fp, W, H, x0 - 2, y0 - 2, pl);
-    }
-    float a[24];
-#pragma unroll
-    for (int s = 0; s < 24; s++) a[s] = la0.wa[s * 64 + lane];
-    Epi8<MODE_A, float, float> epa;
-    epa.load(la0, lane, half);
-    __syncthreads();
-    Epi8<MODE, TIN, TOUT> epi;
-    pair8_first<MODE_A>(pa, pb, a, epa, epi, la);
-    pair8_second<MODE, TIN, TOUT>(pa, pb, W, H, x0, y0, a, epi, fp, fout, la);
-}
-
-template <int MODE, typename TIN, typename TOUT, int MODE_A = kPrelu>
-__global__ __launch_bounds__(kP8NT) void conv8_pair(const float4* __restrict__ fin, long fp, int W, int H,
-                                                  float4* __restrict__ fout, const LayerArgs la0, const LayerArgs la)
-{
-    __shared__ float4 pa[kP8PW * kP8PH];
-    __shared__ float4 pb[kP8PW * kP8PH];
-    const int tiles_x = gridDim.x;
-    const int t = xcd_tile(blockIdx.y * tiles_x + blockIdx.x, tiles_x * gridDim.y);
-    const int ty = t / tiles_x, tx = t - ty * tiles_x;
-    pair8_tile<MODE, TIN, TOUT, MODE_A>(fin, fp, W, H, fout, la0, la, tx * kP8TW, ty * kP8TH, pa, pb);
-}
-
-inline dim3 conv8_pair_grid(int W, int H) { return dim3((W + kP8TW - 1) / kP8TW, (H + kP8TH - 1) / kP8TH); }
 
 // ---- F = 16 or 32: channel tiles ----
 // TW x 16 output pixels per workgroup of NT threads; NI items per wave batch.  The defaults
@@ -564,9 +283,7 @@ __global__ __launch_bounds__(C::NT) void convf_layer(const float4* __restrict__ 
     }
 }
 
-// Grids of the two mappings for a W x H map.
-template <class C = Conv8Tile<>>
-inline dim3 conv8_grid(int W, int H) { return dim3((W + C::TW - 1) / C::TW, (H + C::TH - 1) / C::TH); }
+// Grid for a W x H map.
 template <int F, class C = ConvTile<F>>
 inline dim3 convf_grid(int W, int H) { return dim3((W + C::TW - 1) / C::TW, (H + C::TH - 1) / C::TH); }
 

@@ -10,6 +10,7 @@
 // F-channel f32 maps live in HBM between layers, as for ACNet<8> and ArtCNN.
 #include "acnet_device.hpp"
 #include "acnet_kernels.hpp"
+#include "conv8_rows.hpp"
 #include "conv_layers.hpp"
 
 namespace achip {
@@ -64,10 +65,10 @@ __global__ __launch_bounds__(256) void fsrcnnx_head(const void* __restrict__ src
 long fsrcnnx_feature_pitch(int f, int w) { return (static_cast<long>(w) * f * 4 + 255) / 256 * 256; }
 
 template <int F, int MODE, typename TOUT>
-static void layer(int W, int H, const float4* in, long fp, float4* out, const LayerArgs& la, hipStream_t stream)
+static void layer(int W, int H, const float4* in, long fp, float4* out, const LayerArgs& la, int cus, hipStream_t stream)
 {
     if constexpr (F == 8)
-        hipLaunchKernelGGL((conv8_layer<MODE, float, TOUT>), conv8_grid(W, H), dim3(256), 0, stream, in, fp, W, H, out, la);
+        (void)launch_rows8<kRowsMap, 1, kRelu, MODE, float, TOUT>(rows8_args(in, out, fp, W, H, { la }), cus, stream);
     else
         hipLaunchKernelGGL((convf_layer<F, MODE, TOUT>), convf_grid<F>(W, H), dim3(ConvTile<F>::NT), 0, stream, in, fp, W, H,
                            out, la);
@@ -76,7 +77,7 @@ static void layer(int W, int H, const float4* in, long fp, float4* out, const La
 template <int F, typename TIN, typename TOUT>
 static hipError_t fsrcnnx_pass_t(int blocks, const void* src, long ss, int W, int H, void* dst, long ds,
                                  const float* kernels, const float* biases, const float* alphas, const float* wa,
-                                 const float* w1, char* ws, hipStream_t stream)
+                                 const float* w1, char* ws, int cus, hipStream_t stream)
 {
     const long fp = fsrcnnx_feature_pitch(F, W);
     float4* feat = reinterpret_cast<float4*>(ws);
@@ -107,18 +108,15 @@ static hipError_t fsrcnnx_pass_t(int blocks, const void* src, long ss, int W, in
     int l = 1;
     if constexpr (F == 8) {   // two layers per launch where the first of them is a plain PReLU block
         for (; l + 1 <= blocks; l += 2) {
-            if (l + 1 < blocks)
-                hipLaunchKernelGGL((conv8_pair<kPrelu, float, float>), conv8_pair_grid(W, H), dim3(kP8NT), 0, stream, in, fp, W,
-                                   H, out, body_args(l), body_args(l + 1));
-            else
-                hipLaunchKernelGGL((conv8_pair<kPreluConv1x1, float, float>), conv8_pair_grid(W, H), dim3(kP8NT), 0, stream, in,
-                                   fp, W, H, out, body_args(l), body_args(l + 1));
+            const Rows8 c = rows8_args(in, out, fp, W, H, { body_args(l), body_args(l + 1) });
+            if (l + 1 < blocks) (void)launch_rows8<kRowsMap, 2, kPrelu, kPrelu, float, float>(c, cus, stream);
+            else (void)launch_rows8<kRowsMap, 2, kPrelu, kPreluConv1x1, float, float>(c, cus, stream);
             advance();
         }
     }
     for (; l <= blocks; l++) {
-        if (l < blocks) layer<F, kPrelu, float>(W, H, in, fp, out, body_args(l), stream);
-        else layer<F, kPreluConv1x1, float>(W, H, in, fp, out, body_args(l), stream);
+        if (l < blocks) layer<F, kPrelu, float>(W, H, in, fp, out, body_args(l), cus, stream);
+        else layer<F, kPreluConv1x1, float>(W, H, in, fp, out, body_args(l), cus, stream);
         advance();
     }
     LayerArgs lt{};
@@ -126,16 +124,16 @@ static hipError_t fsrcnnx_pass_t(int blocks, const void* src, long ss, int W, in
     lt.bias = biases + F * (blocks + 2);
     lt.dst = dst;
     lt.ds = ds;
-    layer<F, kShuffle, TOUT>(W, H, in, fp, nullptr, lt, stream);
+    layer<F, kShuffle, TOUT>(W, H, in, fp, nullptr, lt, cus, stream);
     return hipGetLastError();
 }
 
 template <int F>
 static hipError_t fsrcnnx_types(int blocks, int stype, int dtype, const void* src, long ss, int W, int H, void* dst,
                                 long ds, const float* kernels, const float* biases, const float* alphas,
-                                const float* wa, const float* w1, char* ws, hipStream_t stream)
+                                const float* wa, const float* w1, char* ws, int cus, hipStream_t stream)
 {
-#define CALL(TI, TO) fsrcnnx_pass_t<F, TI, TO>(blocks, src, ss, W, H, dst, ds, kernels, biases, alphas, wa, w1, ws, stream)
+#define CALL(TI, TO) fsrcnnx_pass_t<F, TI, TO>(blocks, src, ss, W, H, dst, ds, kernels, biases, alphas, wa, w1, ws, cus, stream)
     switch (stype) {
     case U8: switch (dtype) {
         case U8: return CALL(uint8_t, uint8_t); case U16: return CALL(uint8_t, uint16_t);
@@ -160,38 +158,50 @@ static hipError_t fsrcnnx_types(int blocks, int stype, int dtype, const void* sr
 
 hipError_t launch_fsrcnnx(int f, int blocks, int stype, int dtype, const void* src, long ss, int W, int H, void* dst,
                           long ds, const float* kernels, const float* biases, const float* alphas, const float* wa,
-                          const float* w1, void* workspace, hipStream_t stream)
+                          const float* w1, void* workspace, int cus, hipStream_t stream)
 {
     char* ws = static_cast<char*>(workspace);
     if (f == 8)
-        return fsrcnnx_types<8>(blocks, stype, dtype, src, ss, W, H, dst, ds, kernels, biases, alphas, wa, w1, ws, stream);
+        return fsrcnnx_types<8>(blocks, stype, dtype, src, ss, W, H, dst, ds, kernels, biases, alphas, wa, w1, ws, cus, stream);
     if (f == 16)
-        return fsrcnnx_types<16>(blocks, stype, dtype, src, ss, W, H, dst, ds, kernels, biases, alphas, wa, w1, ws, stream);
+        return fsrcnnx_types<16>(blocks, stype, dtype, src, ss, W, H, dst, ds, kernels, biases, alphas, wa, w1, ws, cus, stream);
     return hipErrorInvalidValue;
 }
 
-// ---- host-side operand packing (layouts read by conv_layers.hpp) ----
+// ---- host-side operand packing (layouts read by conv8_rows.hpp and conv_layers.hpp) ----
 
 void pack_conv8_operands(const float* k, int cout, float* out)
 {
-    // lane l: D/A row i = l % 16 is (output row i / 8, channel i % 8); patch row g = l / 16
-    // feeds output row i / 8 through kernel row ky = g - i / 8
+    // operand ((t * 8 + c) * 3 + ky) * halves + h: output channels 4 h .. 4 h + 3 of tap (ky, t),
+    // input channel c; 16 operands per register, four lanes each
+    const int halves = cout / 4;
+    for (int i = 0; i < kRows8Floats; i++) out[i] = 0.0f;
     for (int t = 0; t < 3; t++)
         for (int c = 0; c < 8; c++)
-            for (int lane = 0; lane < 64; lane++) {
-                const int i = lane % 16, g = lane / 16, n = i % 8, ky = g - i / 8;
-                out[(t * 8 + c) * 64 + lane] = (n < cout && ky >= 0 && ky <= 2) ? k[n * 72 + (ky * 3 + t) * 8 + c] : 0.0f;
+            for (int ky = 0; ky < 3; ky++)
+                for (int n = 0; n < cout; n++) {
+                    const int s = ((t * 8 + c) * 3 + ky) * halves + n / 4;
+                    out[s / 16 * 64 + s % 16 * 4 + n % 4] = k[n * 72 + (ky * 3 + t) * 8 + c];
+                }
+}
+
+void pack_legacy_l0(const float* k, float* out)
+{
+    // operand (t * 3 + ky) * 2 + h, as above
+    for (int i = 0; i < 2 * 64; i++) out[i] = 0.0f;
+    for (int t = 0; t < 3; t++)
+        for (int ky = 0; ky < 3; ky++)
+            for (int n = 0; n < 8; n++) {
+                const int s = (t * 3 + ky) * 2 + n / 4;
+                out[s / 16 * 64 + s % 16 * 4 + n % 4] = k[n * 9 + ky * 3 + t];
             }
 }
 
 void pack_conv8_1x1(const float* k1, float* out)
 {
-    // K step r of lane group g: channel 4 (g & 1) + r of output row g >> 1
-    for (int r = 0; r < 4; r++)
-        for (int lane = 0; lane < 64; lane++) {
-            const int m = lane % 16, g = lane / 16;
-            out[r * 64 + lane] = (m / 8 == (g >> 1)) ? k1[(m % 8) * 8 + 4 * (g & 1) + r] : 0.0f;
-        }
+    // operand i: output channels 4 (i % 2) .., input channel 4 (i / 2 % 2) + i / 4
+    for (int i = 0; i < 16; i++)
+        for (int r = 0; r < 4; r++) out[i * 4 + r] = k1[(4 * (i % 2) + r) * 8 + 4 * (i / 2 % 2) + i / 4];
 }
 
 void pack_convf_operands(const float* k, int f, int cout, float* out)

@@ -96,18 +96,18 @@ ACHIP_API int achip_pass_batch(ACHipNet* net, int precision, int config, int src
                                const ACHipImage* images, int n, void* workspace, size_t workspace_bytes,
                                void* stream);
 
-/* ACNetLegacy's FP32 2x pass layer by layer instead of fused: layers 0-2 in one launch, then
- * layers 3..8 two per launch through 8-channel f32 maps in `workspace`
- * (achip_pass8_workspace_bytes(w, h) bytes, 256-byte aligned, device memory of the net's
- * device, not overlapping src or dst): four launches, each map through HBM once, a one-pixel
- * recompute ring per layer instead of the fused kernel's eight-pixel halo.  Every layer runs
- * the fused FP32 kernel's instructions on the same operands, so the results are its bits.
+/* ACNetLegacy's FP32 2x pass a few layers at a time instead of fused, through 8-channel f32 maps
+ * in `workspace` (achip_pass8_workspace_bytes(w, h) bytes, 256-byte aligned, device memory of the
+ * net's device, not overlapping src or dst): two launches of four layers on small images, four of
+ * two on larger ones (layer 0 with the first), each map through HBM once, a one-pixel recompute
+ * ring per layer and launch instead of the fused kernel's eight-pixel halo.  Every output's
+ * multiply-adds run in the fused FP32 kernel's order, so the results are its bits.
  * The reference's CPU pass runs the layers one by one (CPUProcessor.cpp:1371-1390). */
 ACHIP_API int achip_pass_layers(ACHipNet* net, const void* src, long src_stride, int src_type, int w, int h, void* dst,
                                 long dst_stride, int dst_type, void* workspace, size_t workspace_bytes, void* stream);
 
 /* The layer-split form over a batch of n images of uneven sizes (all src_type -> dst_type),
- * in four launches that each take the tiles of every image (no counterpart in the
+ * in four launches that each take the strips of every image (no counterpart in the
  * reference, whose callers run one pass per image: tools/benchmark/src/Benchmark.cpp:58-63).
  * `workspace`: device memory of achip_pass_batch_layers_bytes(images, n) bytes, 256-byte
  * aligned, the descriptors and every image's two 8-channel f32 maps, not overlapping any
@@ -122,9 +122,9 @@ ACHIP_API int achip_pass_batch_layers(ACHipNet* net, int src_type, int dst_type,
  * the reference's processors run one form, CUDAProcessor.cpp:383-422).  For FP32 ACNetLegacy
  * passes the forms are the fused kernel and the layer-split form of achip_pass_layers, which
  * give the same bits; the choice is the autotuner's for the size class (achip_autotune times
- * both), else a rule measured on MI355X: the fused kernel where its 64 x 32 tiles fit in one
- * round of the device's compute units on an image of more than 256 x 256 pixels, the
- * layer-split form elsewhere (1080p u8: 299 against 328 us).  achip_pass_ws_bytes gives the
+ * both), else a rule measured on MI355X: the fused kernel where its 64 x 32 tiles make just about
+ * one full round of the device's compute units, the layer-split form elsewhere (1080p u8: 213
+ * against 330 us).  achip_pass_ws_bytes gives the
  * workspace bytes the chosen form needs, 0 for the fused kernel and every other net or
  * precision; with a smaller workspace (or none) the pass runs the fused kernel, as achip_pass
  * does.  Workspace rules as for achip_pass_layers. */
