@@ -724,7 +724,7 @@ int achip_pass_net(ACHipNet* net, const void* src, long src_stride, int src_type
     const hipError_t e =
         net->lfamily == kNetArtCNN
             ? achip::launch_artcnn(net->lf, net->lblocks, src_type, dst_type, src, src_stride, w, h, dst, dst_stride, net->lk,
-                                   net->lb, net->lwa, workspace, st)
+                                   net->lb, net->lwa, workspace, compute_units(net->device), st)
             : achip::launch_fsrcnnx(net->lf, net->lblocks, src_type, dst_type, src, src_stride, w, h, dst, dst_stride,
                                     net->lk, net->lb, net->la, net->lwa, net->lw1, workspace, compute_units(net->device), st);
     return e == hipSuccess ? ACHIP_OK : hip_fail(e, "kernel launch");

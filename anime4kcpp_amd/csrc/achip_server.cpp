@@ -303,7 +303,7 @@ hipError_t ACHipServer::pass_launch(int pcfg, int T, const Plane& a, const Plane
                                     achip::compute_units(net->device), st);
     if (net->lfamily == kNetArtCNN)
         return achip::launch_artcnn(net->lf, net->lblocks, T, T, a.ptr, a.stride, a.w, a.h, b.ptr, b.stride, net->lk, net->lb,
-                                    net->lwa, ws.ptr, st);
+                                    net->lwa, ws.ptr, achip::compute_units(net->device), st);
     if (net->lfamily == kNetFSRCNNX)
         return achip::launch_fsrcnnx(net->lf, net->lblocks, T, T, a.ptr, a.stride, a.w, a.h, b.ptr, b.stride, net->lk, net->lb,
                                      net->la, net->lwa, net->lw1, ws.ptr, achip::compute_units(net->device), st);

@@ -131,7 +131,7 @@ hipError_t launch_acnet8_16(int bf16, int blocks, int stype, int dtype, const vo
 long artcnn_feature_pitch(int f, int w);
 hipError_t launch_artcnn(int f, int blocks, int stype, int dtype, const void* src, long ss, int W, int H, void* dst,
                          long ds, const float* kernels, const float* biases, const float* wa, void* workspace,
-                         hipStream_t stream);
+                         int cus, hipStream_t stream);
 
 // FSRCNNX<F> 2x pass, F = 8 or 16 (fsrcnnx.hip): kernels/biases/alphas in the reference
 // layout (device copies); wa the per-lane A operands of the B conv3x3 layers and the F -> 4

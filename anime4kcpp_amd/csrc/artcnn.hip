@@ -1,15 +1,14 @@
 // ArtCNN<F> 2x pass, F = 16 or 32 (core/src/processor/cpu/CPUProcessor.cpp:1519-1546 and the
 // F = 32 twin), layer by layer, FP32 throughout:
 //   head   conv3x3 1 -> F, identity                   -> feat        VALU, one pixel per thread
-//   body   B x conv3x3 F -> F + ReLU                                  convf_layer<kRelu>
-//          conv3x3 F -> F, identity, + feat                           convf_layer<kAddFeat>
-//   tail   conv3x3 F -> 4, identity, pixel shuffle 2x -> dst          convf_layer<kShuffle>
+//   body   B x conv3x3 F -> F + ReLU                                  convf_rows<kRelu>
+//          conv3x3 F -> F, identity, + feat                           convf_rows<kAddFeat>
+//   tail   conv3x3 F -> 4, identity, pixel shuffle 2x -> dst          convf_tail
 // (Backend.hpp:135-215; Common.hpp:116-164, 290-341.)  F-channel f32 maps live in HBM between
-// layers, as for ACNet<8>; the MFMA mapping is convf_layer's (conv_layers.hpp): no MFMA row
-// is padding except in the F -> 4 tail.
+// layers (convf_rows.hpp).
 #include "acnet_device.hpp"
 #include "acnet_kernels.hpp"
-#include "conv_layers.hpp"
+#include "convf_rows.hpp"
 
 namespace achip {
 
@@ -53,7 +52,7 @@ long artcnn_feature_pitch(int f, int w) { return (static_cast<long>(w) * f * 4 +
 
 template <int F, typename TIN, typename TOUT>
 static hipError_t artcnn_pass_t(int blocks, const void* src, long ss, int W, int H, void* dst, long ds,
-                                const float* kernels, const float* biases, const float* wa, char* ws, hipStream_t stream)
+                                const float* kernels, const float* biases, const float* wa, char* ws, int cus, hipStream_t stream)
 {
     const long fp = artcnn_feature_pitch(F, W);
     float4* feat = reinterpret_cast<float4*>(ws);
@@ -61,7 +60,6 @@ static hipError_t artcnn_pass_t(int blocks, const void* src, long ss, int W, int
     float4* m1 = reinterpret_cast<float4*>(ws + 2 * fp * H);
     hipLaunchKernelGGL((artcnn_head<TIN, F>), dim3((W + 63) / 64, (H + 3) / 4), dim3(256), 0, stream, src, ss, W, H, feat,
                        fp, kernels, biases);
-    const dim3 grid = convf_grid<F>(W, H), block(ConvTile<F>::NT);
     const long wl = static_cast<long>(conv_operand_floats(F));   // A-operand floats per layer
     const float4* in = feat;
     float4* out = m0;
@@ -69,7 +67,7 @@ static hipError_t artcnn_pass_t(int blocks, const void* src, long ss, int W, int
         LayerArgs la{};
         la.wa = wa + (l - 1) * wl;
         la.bias = biases + F * l;
-        hipLaunchKernelGGL((convf_layer<F, kRelu, float>), grid, block, 0, stream, in, fp, W, H, out, la);
+        (void)launch_convf<F, kRelu>({ in, out, fp, W, H, 0, la }, cus, stream);
         in = out;
         out = out == m0 ? m1 : m0;
     }
@@ -77,21 +75,20 @@ static hipError_t artcnn_pass_t(int blocks, const void* src, long ss, int W, int
     la.wa = wa + blocks * wl;
     la.bias = biases + F * (blocks + 1);
     la.feat = feat;
-    hipLaunchKernelGGL((convf_layer<F, kAddFeat, float>), grid, block, 0, stream, in, fp, W, H, out, la);
+    (void)launch_convf<F, kAddFeat>({ in, out, fp, W, H, 0, la }, cus, stream);
     LayerArgs lt{};
     lt.wa = wa + (blocks + 1) * wl;
     lt.bias = biases + F * (blocks + 2);
     lt.dst = dst;
     lt.ds = ds;
-    hipLaunchKernelGGL((convf_layer<F, kShuffle, TOUT>), grid, block, 0, stream, out, fp, W, H, nullptr, lt);
-    return hipGetLastError();
+    return launch_convf_tail<F, TOUT>({ out, nullptr, fp, W, H, 0, lt }, cus, stream);
 }
 
 template <int F>
 static hipError_t artcnn_types(int blocks, int stype, int dtype, const void* src, long ss, int W, int H, void* dst, long ds,
-                               const float* kernels, const float* biases, const float* wa, char* ws, hipStream_t stream)
+                               const float* kernels, const float* biases, const float* wa, char* ws, int cus, hipStream_t stream)
 {
-#define CALL(TI, TO) artcnn_pass_t<F, TI, TO>(blocks, src, ss, W, H, dst, ds, kernels, biases, wa, ws, stream)
+#define CALL(TI, TO) artcnn_pass_t<F, TI, TO>(blocks, src, ss, W, H, dst, ds, kernels, biases, wa, ws, cus, stream)
     switch (stype) {
     case U8: switch (dtype) {
         case U8: return CALL(uint8_t, uint8_t); case U16: return CALL(uint8_t, uint16_t);
@@ -116,11 +113,11 @@ static hipError_t artcnn_types(int blocks, int stype, int dtype, const void* src
 
 hipError_t launch_artcnn(int f, int blocks, int stype, int dtype, const void* src, long ss, int W, int H, void* dst,
                          long ds, const float* kernels, const float* biases, const float* wa, void* workspace,
-                         hipStream_t stream)
+                         int cus, hipStream_t stream)
 {
     char* ws = static_cast<char*>(workspace);
-    if (f == 16) return artcnn_types<16>(blocks, stype, dtype, src, ss, W, H, dst, ds, kernels, biases, wa, ws, stream);
-    if (f == 32) return artcnn_types<32>(blocks, stype, dtype, src, ss, W, H, dst, ds, kernels, biases, wa, ws, stream);
+    if (f == 16) return artcnn_types<16>(blocks, stype, dtype, src, ss, W, H, dst, ds, kernels, biases, wa, ws, cus, stream);
+    if (f == 32) return artcnn_types<32>(blocks, stype, dtype, src, ss, W, H, dst, ds, kernels, biases, wa, ws, cus, stream);
     return hipErrorInvalidValue;
 }
 

@@ -26,6 +26,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "acnet_mfma32_item.hpp"   // f32x4m
 #include "conv_layers.hpp"
 #include "stream.hpp"
 

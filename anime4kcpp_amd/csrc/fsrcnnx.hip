@@ -1,17 +1,16 @@
 // FSRCNNX<F> 2x pass, F = 8 or 16 (core/src/processor/cpu/CPUProcessor.cpp:1629-1659 and the
 // F = 16 twin at :1687-1717), layer by layer, FP32 throughout:
 //   head   conv5x5 1 -> F, identity                  -> feat         VALU, one pixel per thread
-//   body   B - 1 x conv3x3 F -> F + PReLU                            conv layer <kPrelu>
-//          conv3x3 F -> F + PReLU, conv1x1 F -> F, * 1 + feat, PReLU conv layer <kPreluConv1x1>
-//   tail   conv3x3 F -> 4, identity, pixel shuffle 2x -> dst         conv layer <kShuffle>
-// (Backend.hpp:225-305; Common.hpp:116-164, 199-341.)  F = 8 runs the 2-row MFMA item
-// (conv8_layer), F = 16 the channel-tile mapping (convf_layer); both fuse the conv1x1 into the
-// last block's epilogue as F/4 x F/16 extra MFMAs fed from the conv3x3's own D registers.
+//   body   B - 1 x conv3x3 F -> F + PReLU                            kPrelu
+//          conv3x3 F -> F + PReLU, conv1x1 F -> F, * 1 + feat, PReLU kPreluConv1x1
+//   tail   conv3x3 F -> 4, identity, pixel shuffle 2x -> dst         kShuffle
+// (Backend.hpp:225-305; Common.hpp:116-164, 199-341.)  F = 8 runs in conv8_rows, F = 16 in
+// convf_rows and convf_tail; the conv1x1 is in the last block's epilogue, fed from the conv3x3's
+// own D registers.
 // F-channel f32 maps live in HBM between layers, as for ACNet<8> and ArtCNN.
 #include "acnet_device.hpp"
 #include "acnet_kernels.hpp"
-#include "conv8_rows.hpp"
-#include "conv_layers.hpp"
+#include "convf_rows.hpp"
 
 namespace achip {
 
@@ -64,14 +63,13 @@ __global__ __launch_bounds__(256) void fsrcnnx_head(const void* __restrict__ src
 
 long fsrcnnx_feature_pitch(int f, int w) { return (static_cast<long>(w) * f * 4 + 255) / 256 * 256; }
 
-template <int F, int MODE, typename TOUT>
+template <int F, int MODE>
 static void layer(int W, int H, const float4* in, long fp, float4* out, const LayerArgs& la, int cus, hipStream_t stream)
 {
     if constexpr (F == 8)
-        (void)launch_rows8<kRowsMap, 1, kRelu, MODE, float, TOUT>(rows8_args(in, out, fp, W, H, { la }), cus, stream);
+        (void)launch_rows8<kRowsMap, 1, kRelu, MODE, float, float>(rows8_args(in, out, fp, W, H, { la }), cus, stream);
     else
-        hipLaunchKernelGGL((convf_layer<F, MODE, TOUT>), convf_grid<F>(W, H), dim3(ConvTile<F>::NT), 0, stream, in, fp, W, H,
-                           out, la);
+        (void)launch_convf<F, MODE>({ in, out, fp, W, H, 0, la }, cus, stream);
 }
 
 template <int F, typename TIN, typename TOUT>
@@ -115,8 +113,8 @@ static hipError_t fsrcnnx_pass_t(int blocks, const void* src, long ss, int W, in
         }
     }
     for (; l <= blocks; l++) {
-        if (l < blocks) layer<F, kPrelu, float>(W, H, in, fp, out, body_args(l), cus, stream);
-        else layer<F, kPreluConv1x1, float>(W, H, in, fp, out, body_args(l), cus, stream);
+        if (l < blocks) layer<F, kPrelu>(W, H, in, fp, out, body_args(l), cus, stream);
+        else layer<F, kPreluConv1x1>(W, H, in, fp, out, body_args(l), cus, stream);
         advance();
     }
     LayerArgs lt{};
@@ -124,8 +122,10 @@ static hipError_t fsrcnnx_pass_t(int blocks, const void* src, long ss, int W, in
     lt.bias = biases + F * (blocks + 2);
     lt.dst = dst;
     lt.ds = ds;
-    layer<F, kShuffle, TOUT>(W, H, in, fp, nullptr, lt, cus, stream);
-    return hipGetLastError();
+    if constexpr (F == 8)
+        return launch_rows8<kRowsMap, 1, kRelu, kShuffle, float, TOUT>(rows8_args(in, nullptr, fp, W, H, { lt }), cus, stream);
+    else
+        return launch_convf_tail<F, TOUT>({ in, nullptr, fp, W, H, 0, lt }, cus, stream);
 }
 
 template <int F>
@@ -168,7 +168,7 @@ hipError_t launch_fsrcnnx(int f, int blocks, int stype, int dtype, const void* s
     return hipErrorInvalidValue;
 }
 
-// ---- host-side operand packing (layouts read by conv8_rows.hpp and conv_layers.hpp) ----
+// ---- host-side operand packing (layouts read by conv8_rows.hpp and convf_rows.hpp) ----
 
 void pack_conv8_operands(const float* k, int cout, float* out)
 {
@@ -206,17 +206,27 @@ void pack_conv8_1x1(const float* k1, float* out)
 
 void pack_convf_operands(const float* k, int f, int cout, float* out)
 {
-    // output channel 16 h + lane % 16, input channel (f / 4) (lane / 16) + q; the F -> 4 tail
-    // has one output tile
-    const int kq = f / 4, mt = cout <= 16 ? 1 : f / 16;
-    for (int p = 0; p < 9; p++)
-        for (int lane = 0; lane < 64; lane++)
+    const int kq = f / 4;
+    if (cout == 4) {   // the tail: operand ((t * kq + q) * 4 + g) * 3 + ky, 16 per register
+        for (int t = 0; t < 3; t++)
             for (int q = 0; q < kq; q++)
-                for (int h = 0; h < mt; h++) {
-                    const int o = 16 * h + lane % 16, c = kq * (lane / 16) + q;
-                    out[(static_cast<size_t>(p) * 64 + lane) * (kq * mt) + q * mt + h] =
-                        o < cout ? k[static_cast<size_t>(o) * 9 * f + p * f + c] : 0.0f;
-                }
+                for (int g = 0; g < 4; g++)
+                    for (int ky = 0; ky < 3; ky++)
+                        for (int n = 0; n < 4; n++) {
+                            const int s = ((t * kq + q) * 4 + g) * 3 + ky;
+                            out[s / 16 * 64 + s % 16 * 4 + n] = k[static_cast<size_t>(n) * 9 * f + (ky * 3 + t) * f + g * kq + q];
+                        }
+        return;
+    }
+    // output channel lane % f, step s of lane group g = lane / f: channel 4 g + s (16 channels),
+    // 8 (2 (s % 2) + g) + s / 2 (32); [tap][s / 4][lane][s % 4]
+    const int steps = f == 16 ? 4 : 16;
+    for (int p = 0; p < 9; p++)
+        for (int s = 0; s < steps; s++)
+            for (int lane = 0; lane < 64; lane++) {
+                const int o = lane % f, g = lane / f, c = f == 16 ? 4 * g + s : 8 * (2 * (s % 2) + g) + s / 2;
+                out[((static_cast<size_t>(p) * (steps / 4) + s / 4) * 64 + lane) * 4 + s % 4] = k[static_cast<size_t>(o) * 9 * f + p * f + c];
+            }
 }
 
 void pack_convf_1x1(const float* k1, int f, float* out)
