@@ -1,6 +1,6 @@
 // ArtCNN<F> 2x pass, F = 16 or 32 (core/src/processor/cpu/CPUProcessor.cpp:1519-1546 and the
 // F = 32 twin), layer by layer, FP32 throughout:
-//   head   conv3x3 1 -> F, identity                   -> feat        VALU, one pixel per thread
+//   head   conv3x3 1 -> F, identity                   -> feat        conv_head
 //   body   B x conv3x3 F -> F + ReLU                                  convf_rows<kRelu>
 //          conv3x3 F -> F, identity, + feat                           convf_rows<kAddFeat>
 //   tail   conv3x3 F -> 4, identity, pixel shuffle 2x -> dst          convf_tail
@@ -8,43 +8,12 @@
 // layers (convf_rows.hpp).
 #include "acnet_device.hpp"
 #include "acnet_kernels.hpp"
+#include "conv_head.hpp"
 #include "convf_rows.hpp"
 
 namespace achip {
 
 #pragma clang fp contract(off)
-
-// ---- head: conv3x3 1 -> F, identity; one pixel per thread, 64 x 4 per workgroup ----
-template <typename TIN, int F>
-__global__ __launch_bounds__(256) void artcnn_head(const void* __restrict__ src, long ss, int W, int H,
-                                                   float4* __restrict__ feat, long fp, const float* __restrict__ k,
-                                                   const float* __restrict__ b)
-{
-    const int x = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int y = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (x >= W || y >= H) return;
-    float r[9];
-#pragma unroll
-    for (int dy = 0; dy < 3; dy++) {
-        const TIN* row = row_ptr<TIN>(src, ss, clampi(y + dy - 1, 0, H - 1));
-#pragma unroll
-        for (int dx = 0; dx < 3; dx++) r[dy * 3 + dx] = to_float<TIN>(row[clampi(x + dx - 1, 0, W - 1)]);
-    }
-    float4* px = reinterpret_cast<float4*>(reinterpret_cast<char*>(feat) + static_cast<long>(y) * fp) + (F / 4) * x;
-#pragma unroll
-    for (int q = 0; q < F / 4; q++) {
-        float o[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int n = 4 * q + i;
-            float s = 0.0f;
-#pragma unroll
-            for (int p = 0; p < 9; p++) s = __fadd_rn(s, __fmul_rn(r[p], k[n * 9 + p]));
-            o[i] = __fadd_rn(s, b[n]);
-        }
-        px[q] = make_float4(o[0], o[1], o[2], o[3]);
-    }
-}
 
 // ---- launch ----
 
@@ -58,8 +27,7 @@ static hipError_t artcnn_pass_t(int blocks, const void* src, long ss, int W, int
     float4* feat = reinterpret_cast<float4*>(ws);
     float4* m0 = reinterpret_cast<float4*>(ws + fp * H);
     float4* m1 = reinterpret_cast<float4*>(ws + 2 * fp * H);
-    hipLaunchKernelGGL((artcnn_head<TIN, F>), dim3((W + 63) / 64, (H + 3) / 4), dim3(256), 0, stream, src, ss, W, H, feat,
-                       fp, kernels, biases);
+    (void)launch_head<TIN, F, 3>({ src, ss, feat, fp, W, H, 0, kernels, biases }, cus, stream);
     const long wl = static_cast<long>(conv_operand_floats(F));   // A-operand floats per layer
     const float4* in = feat;
     float4* out = m0;

@@ -360,7 +360,7 @@ __global__ __launch_bounds__(256, F == 32 ? 2 : 4) void convf_tail(const RowsF c
 inline int convf_heights(long strips, int H, int cus, int most, int lead)
 {
     long best = -1;
-    int rows = H;
+    int rows = 64;   // more strips than four rounds take
     for (int k = 1; k <= most + 2; k++) {
         const int at = k < most ? k : most, rounds = k <= most ? 1 : k == most + 1 ? 2 : 4;
         const long slots = 4L * at * cus, segs = slots * rounds / strips;

@@ -1,6 +1,6 @@
 // FSRCNNX<F> 2x pass, F = 8 or 16 (core/src/processor/cpu/CPUProcessor.cpp:1629-1659 and the
 // F = 16 twin at :1687-1717), layer by layer, FP32 throughout:
-//   head   conv5x5 1 -> F, identity                  -> feat         VALU, one pixel per thread
+//   head   conv5x5 1 -> F, identity                  -> feat         fsrcnnx_head (F = 8), conv_head (16)
 //   body   B - 1 x conv3x3 F -> F + PReLU                            kPrelu
 //          conv3x3 F -> F + PReLU, conv1x1 F -> F, * 1 + feat, PReLU kPreluConv1x1
 //   tail   conv3x3 F -> 4, identity, pixel shuffle 2x -> dst         kShuffle
@@ -10,13 +10,17 @@
 // F-channel f32 maps live in HBM between layers, as for ACNet<8> and ArtCNN.
 #include "acnet_device.hpp"
 #include "acnet_kernels.hpp"
+#include "conv_head.hpp"
 #include "convf_rows.hpp"
 
 namespace achip {
 
 #pragma clang fp contract(off)
 
-// ---- head: conv5x5 1 -> F, identity; one pixel per thread, 64 x 4 per workgroup ----
+// ---- head of F = 8: conv5x5 1 -> 8, identity; one pixel per thread, 64 x 4 per workgroup ----
+// A pixel is two float4 here, and the two stores of a wave fill their lines between them, so a pixel
+// per thread keeps up with conv_head and needs no weights in vector registers: the 1001 x 777 u16
+// pass takes 83.7 us with it and 85.6 with conv_head (F = 16, 1280 x 720: 203 and 197).
 // Taps clamp to the image (Common.hpp:199-225).  The sum follows the reference's FMA order
 // (AVX.hpp:93-124): eight lanes accumulate taps l, l + 8, l + 16 with fused multiply-adds,
 // their tree sum (AVX.hpp:24-30), then tap 24's rounded product, then the bias.
@@ -81,8 +85,11 @@ static hipError_t fsrcnnx_pass_t(int blocks, const void* src, long ss, int W, in
     float4* feat = reinterpret_cast<float4*>(ws);
     float4* m0 = reinterpret_cast<float4*>(ws + fp * H);
     float4* m1 = reinterpret_cast<float4*>(ws + 2 * fp * H);
-    hipLaunchKernelGGL((fsrcnnx_head<TIN, F>), dim3((W + 63) / 64, (H + 3) / 4), dim3(256), 0, stream, src, ss, W, H, feat,
-                       fp, kernels, biases);
+    if constexpr (F == 8)
+        hipLaunchKernelGGL((fsrcnnx_head<TIN, F>), dim3((W + 63) / 64, (H + 3) / 4), dim3(256), 0, stream, src, ss, W, H, feat,
+                           fp, kernels, biases);
+    else
+        (void)launch_head<TIN, F, 5>({ src, ss, feat, fp, W, H, 0, kernels, biases }, cus, stream);
     const long wl = static_cast<long>(conv_operand_floats(F));
     auto body_args = [&](int l) {
         LayerArgs la{};
