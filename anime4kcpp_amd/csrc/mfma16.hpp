@@ -1,5 +1,5 @@
 // The 16-bit MFMA helpers shared by the ACNetLegacy kernel (acnet_stream16.hpp) and the
-// ACNet<8> 16-bit layer kernels (acnet8_mfma16.hip): v_mfma_f32_16x16x32_{f16,bf16} with FP32
+// ACNet<8> 16-bit one (acnet8_stream16.hpp): v_mfma_f32_16x16x32_{f16,bf16} with FP32
 // accumulation, the 16-bit operand vectors, and the round-to-16-bit packing of results.
 #pragma once
 

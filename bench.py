@@ -39,9 +39,10 @@ PEAK_PCIE_GBS = 64.0              # PCIe 5.0 x16, one direction
 FRAMES_PER_VARIANT = 2
 # HBM bytes per 1080p u8 pass of the default configuration of each precision (fp32_split: the
 # layer-split form's four launches together), measured with rocprofv3 --pmc FETCH_SIZE (x2.000)
-# and WRITE_SIZE (x1.000) against a 256 MiB copy (profiles/acnet_fused_1080p_u8.md); counters
+# and WRITE_SIZE (x1.000) against a 256 MiB copy (profiles/acnet_fused_1080p_u8.md, the split form
+# and FP16 profiles/case_kernels.md); counters
 # cannot be read from inside this process.
-MEASURED_TRAFFIC = {"fp32": 11.24e6, "fp16": 11.08e6, "bf16": 11.08e6, "fp32_split": 415.2e6}
+MEASURED_TRAFFIC = {"fp32": 11.24e6, "fp16": 11.22e6, "bf16": 11.22e6, "fp32_split": 466.9e6}
 # bytes per input pixel the layer-split form moves by design: the u8 source, a 32-byte f32 map
 # written by the first launch, read and written by the two middle ones and read by the last,
 # and the four u8 output pixels
@@ -683,8 +684,8 @@ def main():
     kcfg = hip.configs(main_prec)[args.config or 0]
     split = ws_bytes[main_prec] > 0
     if split:
-        path = "achip_pass_ws: layer-split form, 4 launches (legacy_head, conv8_pair x2, conv8_pair + deconv), 8-channel f32 maps in HBM"
-        engine = "FP32 MFMA (v_mfma_f32_16x16x4_f32), FP32 accumulate"
+        path = "achip_pass_ws: layer-split form, 4 launches of conv8_rows (layers 0-2, 3-4, 5-6, 7-8 + deconv), 8-channel f32 maps in HBM"
+        engine = "FP32 MFMA (v_mfma_f32_4x4x1_16b_f32), FP32 accumulate"
         traffic_key = main_prec + "_split"
     else:
         path = {"fp32": "fused FP32 kernel", "fp16": "FP16-MFMA fused kernel", "bf16": "BF16-MFMA fused kernel"}[main_prec]
@@ -728,7 +729,7 @@ def main():
             "unit": "TFLOP/s",
             "frac": round(achieved / peak, 4),
             "traffic": MEASURED_TRAFFIC.get(traffic_key) if args.config is None else None,
-            "traffic_source": "rocprofv3 --pmc FETCH_SIZE/WRITE_SIZE per pass, profiles/acnet_fused_1080p_u8.md",
+            "traffic_source": "rocprofv3 --pmc FETCH_SIZE/WRITE_SIZE per pass, profiles/case_kernels.md",
             "algorithmic_bytes": 5 * W_IN * H_IN,
             "form_bytes": SPLIT_FORM_BYTES_PER_PX * W_IN * H_IN if split else 5 * W_IN * H_IN,
             "mean_pass_us": round(mean_pass_s * 1e6, 2),
