@@ -1156,13 +1156,13 @@ int achip_pass_batch_layers(ACHipNet* net, int src_type, int dst_type, const ACH
         const long fp = achip::acnet8_feature_pitch(im.w);
         auto* m0 = reinterpret_cast<float4*>(ws + offsets[i]);
         auto* m1 = reinterpret_cast<float4*>(ws + offsets[i] + static_cast<size_t>(fp) * im.h);
-        const int cols = achip::legacy_batch_cols();
-        desc[i] = achip::SplitDesc{ im.src, im.dst, m0, m1, im.src_stride, im.dst_stride, fp, im.w, im.h, (im.w + cols - 1) / cols, 0 };
+        desc[i] = achip::SplitDesc{ im.src, im.dst, m0, m1, im.src_stride, im.dst_stride, fp, im.w, im.h, 0, 0 };
     }
-    const int rows = achip::legacy_batch_rows(desc.data(), n, compute_units(net->device));
+    const achip::BatchSplit sp = achip::legacy_batch_split(desc.data(), n, compute_units(net->device));
     for (achip::SplitDesc& d : desc) {
         d.first_tile = static_cast<int>(total);
-        total += static_cast<long>(d.tiles_x) * ((d.h + rows - 1) / rows);
+        d.tiles_x = (d.w + sp.cols - 1) / sp.cols;
+        total += static_cast<long>(d.tiles_x) * ((d.h + sp.rows - 1) / sp.rows);
         if (total > (1L << 30)) return fail(ACHIP_EINVAL, "batch too large (%ld tiles)", total);
     }
     // the maps and descriptors are written by the launches: no image may overlap them, and no
@@ -1179,7 +1179,7 @@ int achip_pass_batch_layers(ACHipNet* net, int src_type, int dst_type, const ACH
                                   hipMemcpyHostToDevice, st);
     if (e == hipSuccess)
         e = achip::launch_legacy_split_batch(src_type, dst_type, reinterpret_cast<const achip::SplitDesc*>(workspace), n,
-                                             static_cast<int>(total), rows, net->wts, net->wa4, st);
+                                             static_cast<int>(total), sp, net->wts, net->wa4, st);
     return e == hipSuccess ? ACHIP_OK : hip_fail(e, "kernel launch");
 }
 

@@ -8,6 +8,8 @@
 // Features between launches are 8-channel f32 maps in HBM (32 bytes per pixel, rows padded to 256
 // bytes).  Borders replicate the edge pixel at every layer, as the reference's clamped taps
 // (Common.hpp:120-160) do.
+#include <algorithm>
+#include <cmath>
 #include <utility>
 
 #include "acnet_device.hpp"
@@ -149,53 +151,70 @@ static hipError_t legacy_split_t(const void* src, long ss, int W, int H, void* d
 }
 
 // ---- the layer-split form over a batch of images: every launch takes the strips of all of them,
-// each image with its own two maps; layer 0 with layers 1-2, then two layers per launch, all cut
-// into the first launch's columns ----
+// each image with its own two maps, all launches cut into the first one's columns: layer 0 with
+// layers 1-2 and then two layers per launch, or layer 0 with layers 1-4 and then 5-8.
+// 64 images of sides 128-2048 (30.7 Mpix): 3.04 ms, 4.06 before; three of 96 kpix in all 42 us, 58 ----
 
-int legacy_batch_cols() { return rows8_out<kRowsLegacy, 2>(); }
-
-// The height whose strips over all images take the fewest steps per CU (four strips at a time on
-// each), plus half a strip's for the uneven end.
-int legacy_batch_rows(const SplitDesc* desc, int n, int cus)
+// What a launch of n strips of `rows` rows takes: a strip has two steps per layer after the first and
+// about three to start, a step takes a fixed part and one for every layer and strip on the CU, and
+// strips beyond one round of the CUs come in where others end, half a round late at the end.
+// Measured, layers per launch / rows: 300 x 143 .. 483 x 409, four images, 2 / 12 88 us, 2 / 20 98,
+// 4 / 20 88, 4 / 40 92 (62 x 16 tiles before: 91); eight of 250 x 200 2 / 8 81, 2 / 20 97, 4 / 18 83,
+// 4 / 40 93; four of 512 x 512 2 / 20 148, 2 / 32 173, 4 / 28 159 (before: 183).
+static double batch_cost(double n, int rows, int layers, int per_cu, int cus)
 {
-    double best = -1.0;
-    int rows = 32;
-    for (int r : { 8, 16, 24, 32, 48, 64, 96, 128, 192, 256 }) {
-        double steps = 0.0;
-        for (int i = 0; i < n; i++) steps += desc[i].tiles_x * (desc[i].h / 2 + (desc[i].h + r - 1) / r * 3.0);
-        const double cost = steps / (4.0 * cus) + 0.5 * (r / 2 + 4);
-        if (best < 0.0 || cost < best) {
-            best = cost;
-            rows = r;
+    const double at = std::min<double>(per_cu, std::ceil(n / cus)), rounds = n / (at * cus);
+    return (rows / 2 + 2 * (layers - 1) + 3) * (4.0 + at * layers) * (rounds <= 1.0 ? 1.0 : rounds + 0.5);
+}
+
+BatchSplit legacy_batch_split(const SplitDesc* desc, int n, int cus)
+{
+    BatchSplit best{ rows8_out<kRowsLegacy, 2>(), 32, 2 };
+    double least = -1.0;
+    for (int layers : { 2, 4 }) {
+        const int cols = layers == 2 ? rows8_out<kRowsLegacy, 2>() : rows8_out<kRowsLegacy, 4>();
+        const int per_cu = layers == 2 ? rows8_per_cu<kRowsMap, 2>() : rows8_per_cu<kRowsMap, 4>();
+        for (int r : { 4, 6, 8, 10, 12, 16, 20, 24, 28, 32, 40, 48, 64, 80, 96, 128, 192, 256 }) {
+            double strips = 0.0;
+            for (int i = 0; i < n; i++)
+                strips += static_cast<double>((desc[i].w + cols - 1) / cols) * ((desc[i].h + r - 1) / r);
+            const double cost = 8 / layers * batch_cost(strips, r, layers, per_cu, cus);
+            if (least < 0.0 || cost < least) {
+                least = cost;
+                best = { cols, r, layers };
+            }
         }
     }
-    return rows;
+    return best;
+}
+
+template <int HEAD, int NL, int MODE, typename TIN, typename TOUT>
+static void batch_launch(const SplitDesc* desc, int n, int total, const BatchSplit& sp, int first, const float* wts, const float* wa4,
+                         hipStream_t stream)
+{
+    Rows8 c{};
+    c.w0 = wa4;
+    c.b0 = wts + kOffB0;
+    c.rows = sp.rows;
+    for (int i = 0; i < NL; i++) c.la[i] = legacy_layer(first + i, wts, wa4, nullptr, 0);
+    // the first launch writes map 0 (it reads no map), then 0 -> 1 -> 0 -> the outputs
+    hipLaunchKernelGGL((conv8_rows_batch<HEAD, NL, kRelu, MODE, TIN, TOUT>), dim3(total), dim3(rows8_threads<HEAD, NL>()), 0, stream,
+                       desc, n, total, sp.cols, ((first - 1) / NL & 1) == 0, c);
 }
 
 template <typename TIN, typename TOUT>
-static hipError_t legacy_split_batch_t(const SplitDesc* desc, int n, int total, int rows, const float* wts, const float* wa4,
+static hipError_t legacy_split_batch_t(const SplitDesc* desc, int n, int total, const BatchSplit& sp, const float* wts, const float* wa4,
                                        hipStream_t stream)
 {
-    const int out = legacy_batch_cols();
-    const dim3 grid(total);
-    auto args = [&](int l) {
-        Rows8 c{};
-        c.w0 = wa4;
-        c.b0 = wts + kOffB0;
-        c.rows = rows;
-        c.la[0] = legacy_layer(l, wts, wa4, nullptr, 0);
-        c.la[1] = legacy_layer(l + 1, wts, wa4, nullptr, 0);
-        return c;
-    };
-    // the first launch writes map 0 (it reads no map), then 0 -> 1 -> 0 -> the outputs
-    hipLaunchKernelGGL((conv8_rows_batch<kRowsLegacy, 2, kRelu, kRelu, TIN, float>), grid, dim3(rows8_threads<kRowsLegacy, 2>()), 0, stream,
-                       desc, n, total, out, 1, args(1));
-    hipLaunchKernelGGL((conv8_rows_batch<kRowsMap, 2, kRelu, kRelu, float, float>), grid, dim3(rows8_threads<kRowsMap, 2>()), 0, stream,
-                       desc, n, total, out, 0, args(3));
-    hipLaunchKernelGGL((conv8_rows_batch<kRowsMap, 2, kRelu, kRelu, float, float>), grid, dim3(rows8_threads<kRowsMap, 2>()), 0, stream,
-                       desc, n, total, out, 1, args(5));
-    hipLaunchKernelGGL((conv8_rows_batch<kRowsMap, 2, kRelu, kReluDeconv, float, TOUT>), grid, dim3(rows8_threads<kRowsMap, 2>()), 0, stream,
-                       desc, n, total, out, 0, args(7));
+    if (sp.layers == 4) {
+        batch_launch<kRowsLegacy, 4, kRelu, TIN, float>(desc, n, total, sp, 1, wts, wa4, stream);
+        batch_launch<kRowsMap, 4, kReluDeconv, float, TOUT>(desc, n, total, sp, 5, wts, wa4, stream);
+    } else {
+        batch_launch<kRowsLegacy, 2, kRelu, TIN, float>(desc, n, total, sp, 1, wts, wa4, stream);
+        batch_launch<kRowsMap, 2, kRelu, float, float>(desc, n, total, sp, 3, wts, wa4, stream);
+        batch_launch<kRowsMap, 2, kRelu, float, float>(desc, n, total, sp, 5, wts, wa4, stream);
+        batch_launch<kRowsMap, 2, kReluDeconv, float, TOUT>(desc, n, total, sp, 7, wts, wa4, stream);
+    }
     return hipGetLastError();
 }
 
@@ -231,11 +250,11 @@ hipError_t launch_legacy_split(int stype, int dtype, const void* src, long ss, i
 #undef CALL
 }
 
-hipError_t launch_legacy_split_batch(int stype, int dtype, const SplitDesc* desc, int n, int total, int rows, const float* wts,
-                                     const float* wa4, hipStream_t stream)
+hipError_t launch_legacy_split_batch(int stype, int dtype, const SplitDesc* desc, int n, int total, const BatchSplit& sp,
+                                     const float* wts, const float* wa4, hipStream_t stream)
 {
     if (n <= 0 || total <= 0) return hipSuccess;
-#define CALL(TI, TO) legacy_split_batch_t<TI, TO>(desc, n, total, rows, wts, wa4, stream)
+#define CALL(TI, TO) legacy_split_batch_t<TI, TO>(desc, n, total, sp, wts, wa4, stream)
     ACHIP_TYPES(CALL)
 #undef CALL
 }

@@ -109,11 +109,14 @@ constexpr int kRows8L0Floats = 2 * 64, kRows8Floats = 9 * 64;
 hipError_t launch_legacy_split(int stype, int dtype, const void* src, long ss, int W, int H, void* dst, long ds,
                                const float* wts, const float* wa4, void* workspace, int cus, hipStream_t stream);
 // The same for n images (one element type pair) in launches over the strips of all of them,
-// `total` in all, of legacy_batch_cols() columns and `rows` rows; desc is device memory.
-int legacy_batch_cols();
-int legacy_batch_rows(const SplitDesc* desc, int n, int cus);
-hipError_t launch_legacy_split_batch(int stype, int dtype, const SplitDesc* desc, int n, int total, int rows, const float* wts,
-                                     const float* wa4, hipStream_t stream);
+// `total` in all, cut as legacy_batch_split says for the images' widths and heights (columns and
+// rows of a strip, layers per launch: two or four); desc is device memory.
+struct BatchSplit {
+    int cols, rows, layers;
+};
+BatchSplit legacy_batch_split(const SplitDesc* desc, int n, int cus);
+hipError_t launch_legacy_split_batch(int stype, int dtype, const SplitDesc* desc, int n, int total, const BatchSplit& sp,
+                                     const float* wts, const float* wa4, hipStream_t stream);
 
 // ACNet<8> 2x pass with the conv3x3 layers on 16-bit MFMA, streamed (acnet8_stream16.hpp):
 // bf16 = 0 FP16, 1 BF16 operands; wa16 that type's per-lane A operands of the blocks and the

@@ -218,8 +218,8 @@ class Net:
         return dsts
 
     def upscale_batch_layers(self, srcs, dsts=None, stream=None, workspace=None, out_dtype=None):
-        """FP32 2x passes of many images (same element types) in the layer-split form, four
-        launches over the strips of all of them (achip_pass_batch_layers); outputs are the
+        """FP32 2x passes of many images (same element types) in the layer-split form, two or
+        four launches over the strips of all of them (achip_pass_batch_layers); outputs are the
         fused kernel's bits.  workspace: a device tensor of batch_layers_bytes(srcs) bytes, or
         None to allocate one.  Returns the list of outputs."""
         import torch

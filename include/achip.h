@@ -107,7 +107,7 @@ ACHIP_API int achip_pass_layers(ACHipNet* net, const void* src, long src_stride,
                                 long dst_stride, int dst_type, void* workspace, size_t workspace_bytes, void* stream);
 
 /* The layer-split form over a batch of n images of uneven sizes (all src_type -> dst_type),
- * in four launches that each take the strips of every image (no counterpart in the
+ * in two or four launches that each take the strips of every image (no counterpart in the
  * reference, whose callers run one pass per image: tools/benchmark/src/Benchmark.cpp:58-63).
  * `workspace`: device memory of achip_pass_batch_layers_bytes(images, n) bytes, 256-byte
  * aligned, the descriptors and every image's two 8-channel f32 maps, not overlapping any

@@ -60,3 +60,14 @@ def test_fsrcnnx8_edges(cuda, w, h):
     got = net.upscale(torch.from_numpy(x).to(cuda)).cpu().numpy()
     assert np.abs(got - OL.oracle_fsrcnnx(x, k, b, a, f, blocks)).max() <= 1e-5
     net.close()
+
+
+@pytest.mark.parametrize("dims", [[(56, 5), (57, 1), (113, 20), (3, 40)], [(512, 300)] * 3, [(61, 2100), (240, 256), (7, 9)], [(700, 512)] * 4])
+def test_batch_splits(cuda, dims):
+    """Small batches take four layers per launch, larger ones two: each image is its own fused pass."""
+    net = hip.Net("hdn3", 0)
+    srcs = [torch.from_numpy(synth.flat_shaded(990 + i + w, w, h, dtype=np.uint8)).to(cuda) for i, (w, h) in enumerate(dims)]
+    out = net.upscale_batch_layers(srcs)
+    for s, d in zip(srcs, out):
+        assert torch.equal(d, net.upscale(s, config=0))
+    net.close()
