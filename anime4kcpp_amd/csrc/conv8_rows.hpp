@@ -260,12 +260,13 @@ struct RowsMapFeed {
     long fp;
     int H, row, tid;
     unsigned off = 0;
-    __device__ __forceinline__ RowsMapFeed(const RowsIo& c, int xs, int row0, int tid_) : fin(reinterpret_cast<const char*>(c.fin)), fp(c.fp), H(c.H), row(row0), tid(tid_)
+    __device__ __forceinline__ RowsMapFeed(const RowsIo& c, int xs, int row0, int tid_)
+        : fin(reinterpret_cast<const char*>(c.fin) + 32L * clampi(xs, 0, c.W - 1)), fp(c.fp), H(c.H), row(row0), tid(tid_)
     {
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const int e = min(tid + k * NT, N - 1), f = e % (2 * kR8In);
-            o[k] = 32 * clampi(xs + (f >> 1), 0, c.W - 1) + 16 * (f & 1);
+            o[k] = 32 * (clampi(xs + (f >> 1), 0, c.W - 1) - clampi(xs, 0, c.W - 1)) + 16 * (f & 1);
             at[k] = e / (2 * kR8In) * kR8Row + (f & 1) * kR8Plane + (f >> 1) * 16;
         }
     }

@@ -93,15 +93,16 @@ __global__ __launch_bounds__(256, WAVES) void convf_rows(const RowsF c)
     const int ty = id / strips, x0 = (id - ty * strips) * kStripF;
     const int y0 = ty * c.rows, y1 = min(y0 + c.rows, c.H);
 
-    // this lane's channels of patch columns 0-2, one input row
+    // this lane's channels of patch columns 0-2, one input row, from the strip's first input column on
+    const int xb = max(x0 - 1, 0);
     int off[3][NB];
 #pragma unroll
     for (int d = 0; d < 3; d++)
 #pragma unroll
-        for (int n = 0; n < NB; n++) off[d][n] = clampi(x0 + PX * n + j + d - 1, 0, c.W - 1) * (4 * F) + g * M::kIn;
+        for (int n = 0; n < NB; n++) off[d][n] = (clampi(x0 + PX * n + j + d - 1, 0, c.W - 1) - xb) * (4 * F) + g * M::kIn;
     f32x4m b[3][NB][NQ];
     auto fetch = [&](int d, int r) {
-        const char* row = reinterpret_cast<const char*>(c.fin) + static_cast<long>(clampi(r, 0, c.H - 1)) * c.fp;
+        const char* row = reinterpret_cast<const char*>(c.fin) + static_cast<long>(clampi(r, 0, c.H - 1)) * c.fp + static_cast<long>(xb) * (4 * F);
 #pragma unroll
         for (int n = 0; n < NB; n++)
 #pragma unroll
@@ -142,12 +143,13 @@ __global__ __launch_bounds__(256, WAVES) void convf_rows(const RowsF c)
             for (int i = 0; i < 4; i++) a[p][4 * v + i] = f[i];
         }
 
-    // a row of the output or the skip map as a buffer of this row's bytes: the stores of lanes right
+    // the strip's part of a row of the output or the skip map as a buffer: the stores of lanes right
     // of the image fall outside it and are dropped, with no branch to end the loads' overlap
-    const int px = (x0 + j) * (4 * F) + g * M::kOut, row_bytes = c.W * (4 * F);
+    const int px = j * (4 * F) + g * M::kOut, row_bytes = min(c.W - x0, kStripF) * (4 * F);
     auto row_of = [&](const float4* map, int y) {
         return __builtin_amdgcn_make_buffer_rsrc(
-            reinterpret_cast<char*>(const_cast<float4*>(map)) + static_cast<long>(y) * c.fp, 0, row_bytes, 0x00020000);
+            reinterpret_cast<char*>(const_cast<float4*>(map)) + static_cast<long>(y) * c.fp + static_cast<long>(x0) * (4 * F), 0, row_bytes,
+            0x00020000);
     };
     f32x4m feat[NB][NQ];
     auto ahead = [&](int y) {
@@ -301,16 +303,17 @@ __global__ __launch_bounds__(256, F == 32 ? 2 : 4) void convf_tail(const RowsF c
     if (y0 >= c.H) return;
     char* const buf = reinterpret_cast<char*>(lds[wave]);
 
+    const int xb = max(x0 - 1, 0);   // the first input column
     int at[K], off[K];
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const int e = min(lane + 64 * k, N - 1);
-        off[k] = clampi(x0 - 1 + e / NQ, 0, c.W - 1) * (4 * F) + e % NQ * 16;
+        off[k] = (clampi(x0 - 1 + e / NQ, 0, c.W - 1) - xb) * (4 * F) + e % NQ * 16;
         at[k] = e % NQ * PITCH + e / NQ * 16;
     }
     f32x4m v[K];
     auto fetch = [&](int r) {
-        const char* row = reinterpret_cast<const char*>(c.fin) + static_cast<long>(clampi(r, 0, c.H - 1)) * c.fp;
+        const char* row = reinterpret_cast<const char*>(c.fin) + static_cast<long>(clampi(r, 0, c.H - 1)) * c.fp + static_cast<long>(xb) * (4 * F);
 #pragma unroll
         for (int k = 0; k < K; k++) v[k] = *reinterpret_cast<const f32x4m*>(row + off[k]);
     };

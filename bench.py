@@ -231,7 +231,7 @@ def batched_uneven(nets, prec, seed=2024, n=64, streams=None):
         # the serving section's streams share (4 per process by default)
         sts = list(streams[:2]) if streams and len(streams) >= 2 else [torch.cuda.current_stream(dev), torch.cuda.Stream(dev)]
         st = sts[0].cuda_stream
-        sweep_ms["62x16/256thr/mfma/layer-split (per image)"] = round(
+        sweep_ms["64-column strips/mfma/layer-split (per image)"] = round(
             timed(lambda: [layer_split_pass(net, s, d, lws[0], st) for s, d in zip(srcs, dsts)]) * 1e3, 3)
 
         def two_streams():
@@ -243,9 +243,9 @@ def batched_uneven(nets, prec, seed=2024, n=64, streams=None):
             ev2 = torch.cuda.Event()
             ev2.record(sts[1])
             sts[0].wait_event(ev2)
-        sweep_ms["62x16/256thr/mfma/layer-split (per image, two streams)"] = round(timed(two_streams) * 1e3, 3)
+        sweep_ms["64-column strips/mfma/layer-split (per image, two streams)"] = round(timed(two_streams) * 1e3, 3)
         bws = torch.empty(net.batch_layers_bytes(srcs), dtype=torch.uint8, device=dev)
-        sweep_ms["62x16/256thr/mfma/layer-split batched (4 launches over all images)"] = round(
+        sweep_ms["64-column strips/mfma/layer-split batched (2 or 4 launches over all images)"] = round(
             timed(lambda: net.upscale_batch_layers(srcs, dsts, workspace=bws)) * 1e3, 3)
         del bws
     out = {
@@ -255,7 +255,7 @@ def batched_uneven(nets, prec, seed=2024, n=64, streams=None):
         "autotune_sweep_ms": sweep_ms,
         "chosen_config": best,
     }
-    key = "62x16/256thr/mfma/layer-split batched (4 launches over all images)"
+    key = "64-column strips/mfma/layer-split batched (2 or 4 launches over all images)"
     if key in sweep_ms:
         tl = sweep_ms[key] / 1e3
         out["layer_split_batched"] = {"images_per_s": round(n / tl, 1), "mpix_per_s": round(out_mpix / tl, 1),
