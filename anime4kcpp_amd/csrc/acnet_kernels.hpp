@@ -129,7 +129,8 @@ hipError_t launch_acnet8_16(int bf16, int blocks, int stype, int dtype, const vo
 
 // ArtCNN<F> 2x pass, F = 16 or 32 (artcnn.hip): kernels/biases in the reference layout
 // (device copies), wa the per-lane A operands of the B body layers, the residual layer and
-// the F -> 4 tail, 9 * 64 * (F/4) * (F/16) floats each ([tap][lane][K step][channel tile]).
+// the F -> 4 tail, conv_operand_floats(F) floats each (pack_convf_operands); cus the device's
+// compute units.
 // Workspace: 3 * artcnn_feature_pitch(F, W) * H bytes (head features and two maps).
 long artcnn_feature_pitch(int f, int w);
 hipError_t launch_artcnn(int f, int blocks, int stype, int dtype, const void* src, long ss, int W, int H, void* dst,
@@ -149,8 +150,8 @@ hipError_t launch_fsrcnnx(int f, int blocks, int stype, int dtype, const void* s
 // Host-side packing of the A operands the layer kernels read.  F = 8 (conv8_rows.hpp), conv3x3
 // 8 -> cout (8 or 4) in kRows8Floats floats, ACNetLegacy's layer 0 in kRows8L0Floats, conv1x1
 // 8 -> 8 in 64: 16 operands of four output channels per register.
-// F = 16 or 32 (channel tiles), conv3x3 F -> F: [tap][lane][q * F/16 + h]; F -> 4 (the tail,
-// one output tile): [tap][lane][q];
+// F = 16 or 32 (convf_rows.hpp), conv3x3 F -> F: [tap][step / 4][lane][step % 4]; F -> 4 (the
+// tail): 16 operands of the four outputs per register;
 // conv1x1 F -> F: [4 h + r][lane][h2].  k in the reference layout k[n][tap][c].
 void pack_conv8_operands(const float* k, int cout, float* out);
 void pack_legacy_l0(const float* k, float* out);
