@@ -27,23 +27,26 @@ static hipError_t artcnn_pass_t(int blocks, const void* src, long ss, int W, int
     float4* feat = reinterpret_cast<float4*>(ws);
     float4* m0 = reinterpret_cast<float4*>(ws + fp * H);
     float4* m1 = reinterpret_cast<float4*>(ws + 2 * fp * H);
-    (void)launch_head<TIN, F, 3>({ src, ss, feat, fp, W, H, 0, kernels, biases }, cus, stream);
+    // every launch's error is its own (the helpers read hipGetLastError): the pass ends at the first
+    hipError_t e = launch_head<TIN, F, 3>({ src, ss, feat, fp, W, H, 0, kernels, biases }, cus, stream);
     const long wl = static_cast<long>(conv_operand_floats(F));   // A-operand floats per layer
     const float4* in = feat;
     float4* out = m0;
-    for (int l = 1; l <= blocks; l++) {         // body: F -> F + ReLU
+    for (int l = 1; l <= blocks && e == hipSuccess; l++) {   // body: F -> F + ReLU
         LayerArgs la{};
         la.wa = wa + (l - 1) * wl;
         la.bias = biases + F * l;
-        (void)launch_convf<F, kRelu>({ in, out, fp, W, H, 0, la }, cus, stream);
+        e = launch_convf<F, kRelu>({ in, out, fp, W, H, 0, la }, cus, stream);
         in = out;
         out = out == m0 ? m1 : m0;
     }
+    if (e != hipSuccess) return e;
     LayerArgs la{};
     la.wa = wa + blocks * wl;
     la.bias = biases + F * (blocks + 1);
     la.feat = feat;
-    (void)launch_convf<F, kAddFeat>({ in, out, fp, W, H, 0, la }, cus, stream);
+    e = launch_convf<F, kAddFeat>({ in, out, fp, W, H, 0, la }, cus, stream);
+    if (e != hipSuccess) return e;
     LayerArgs lt{};
     lt.wa = wa + (blocks + 1) * wl;
     lt.bias = biases + F * (blocks + 2);

@@ -67,15 +67,6 @@ __global__ __launch_bounds__(256) void fsrcnnx_head(const void* __restrict__ src
 
 long fsrcnnx_feature_pitch(int f, int w) { return (static_cast<long>(w) * f * 4 + 255) / 256 * 256; }
 
-template <int F, int MODE>
-static void layer(int W, int H, const float4* in, long fp, float4* out, const LayerArgs& la, int cus, hipStream_t stream)
-{
-    if constexpr (F == 8)
-        (void)launch_rows8<kRowsMap, 1, kRelu, MODE, float, float>(rows8_args(in, out, fp, W, H, { la }), cus, stream);
-    else
-        (void)launch_convf<F, MODE>({ in, out, fp, W, H, 0, la }, cus, stream);
-}
-
 template <int F, typename TIN, typename TOUT>
 static hipError_t fsrcnnx_pass_t(int blocks, const void* src, long ss, int W, int H, void* dst, long ds,
                                  const float* kernels, const float* biases, const float* alphas, const float* wa,
@@ -85,11 +76,15 @@ static hipError_t fsrcnnx_pass_t(int blocks, const void* src, long ss, int W, in
     float4* feat = reinterpret_cast<float4*>(ws);
     float4* m0 = reinterpret_cast<float4*>(ws + fp * H);
     float4* m1 = reinterpret_cast<float4*>(ws + 2 * fp * H);
-    if constexpr (F == 8)
+    // every launch's error is its own (the helpers read hipGetLastError): the pass ends at the first
+    hipError_t e = hipSuccess;
+    if constexpr (F == 8) {
         hipLaunchKernelGGL((fsrcnnx_head<TIN, F>), dim3((W + 63) / 64, (H + 3) / 4), dim3(256), 0, stream, src, ss, W, H, feat,
                            fp, kernels, biases);
-    else
-        (void)launch_head<TIN, F, 5>({ src, ss, feat, fp, W, H, 0, kernels, biases }, cus, stream);
+        e = hipGetLastError();
+    } else {
+        e = launch_head<TIN, F, 5>({ src, ss, feat, fp, W, H, 0, kernels, biases }, cus, stream);
+    }
     const long wl = static_cast<long>(conv_operand_floats(F));
     auto body_args = [&](int l) {
         LayerArgs la{};
@@ -110,20 +105,25 @@ static hipError_t fsrcnnx_pass_t(int blocks, const void* src, long ss, int W, in
         in = out;
         out = out == m0 ? m1 : m0;
     };
-    int l = 1;
-    if constexpr (F == 8) {   // two layers per launch where the first of them is a plain PReLU block
-        for (; l + 1 <= blocks; l += 2) {
-            const Rows8 c = rows8_args(in, out, fp, W, H, { body_args(l), body_args(l + 1) });
-            if (l + 1 < blocks) (void)launch_rows8<kRowsMap, 2, kPrelu, kPrelu, float, float>(c, cus, stream);
-            else (void)launch_rows8<kRowsMap, 2, kPrelu, kPreluConv1x1, float, float>(c, cus, stream);
+    if constexpr (F == 8) {   // two layers per launch, the last one alone where the count is odd
+        for (int l = 1; l <= blocks && e == hipSuccess; l += 2) {
+            if (l == blocks) {
+                e = launch_rows8<kRowsMap, 1, kRelu, kPreluConv1x1, float, float>(rows8_args(in, out, fp, W, H, { body_args(l) }), cus, stream);
+            } else {
+                const Rows8 c = rows8_args(in, out, fp, W, H, { body_args(l), body_args(l + 1) });
+                e = l + 1 < blocks ? launch_rows8<kRowsMap, 2, kPrelu, kPrelu, float, float>(c, cus, stream)
+                                   : launch_rows8<kRowsMap, 2, kPrelu, kPreluConv1x1, float, float>(c, cus, stream);
+            }
+            advance();
+        }
+    } else {
+        for (int l = 1; l <= blocks && e == hipSuccess; l++) {
+            const RowsF c{ in, out, fp, W, H, 0, body_args(l) };
+            e = l < blocks ? launch_convf<F, kPrelu>(c, cus, stream) : launch_convf<F, kPreluConv1x1>(c, cus, stream);
             advance();
         }
     }
-    for (; l <= blocks; l++) {
-        if (l < blocks) layer<F, kPrelu>(W, H, in, fp, out, body_args(l), cus, stream);
-        else layer<F, kPreluConv1x1>(W, H, in, fp, out, body_args(l), cus, stream);
-        advance();
-    }
+    if (e != hipSuccess) return e;
     LayerArgs lt{};
     lt.wa = wa + blocks * wl;
     lt.bias = biases + F * (blocks + 2);
