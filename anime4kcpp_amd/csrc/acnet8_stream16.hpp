@@ -33,6 +33,21 @@ constexpr int kS8MaxWaves = 12;
 // also the loader) 9, behind a map (one loader wave) 10, so at most 10 rings, two workgroups
 // per CU.
 constexpr int kS8L0Waves = 3, kS8MaxImg = 9, kS8MaxMap = 10;
+
+// The last layer's wave takes whole segments of 16 pixels: five where a strip has more than 64 output
+// columns, else four.  Lane j's patch in segment i starts at pixel n - 1 + j + 16 i, so with five the
+// lanes past the strip's columns read up to pixel n + 80 of a row of 80 (and store nothing).
+constexpr int s8_segments(int n) { return kSCols - 2 * n > 64 ? 5 : 4; }
+constexpr int s8_last_pixel(int n) { return n - 1 + 15 + 16 * (s8_segments(n) - 1) + 2; }
+// LDS of a launch of n layers: a pixel, the rings, then a pixel and the source rows (image head), or
+// the pixels that the last segment reads past the last ring's last row.
+constexpr unsigned s8_lds_bytes(bool img, int n)
+{
+    return 16 + n * kSRingBytes +
+           (img ? 16 + kSImgBytes : 16u * static_cast<unsigned>(s8_last_pixel(n) >= kSCols ? s8_last_pixel(n) + 1 - kSCols : 1));
+}
+static_assert(16 * (s8_last_pixel(7) + 1 - kSCols) <= 16 + static_cast<int>(kSImgBytes), "with an image head that is the source rows");
+
 enum S8Role : unsigned char { kS8L0 = 1, kS8Last = 4, kS8Layer = 8 };   // kS8L0 + part, kS8Layer + layer
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -296,7 +311,7 @@ template <typename T16, typename TIN, typename TOUT, bool IMG, bool FINAL>
 __global__ __launch_bounds__(64 * kS8MaxWaves, 6) void acnet8_stream16(const Chunk8 c)
 {
     extern __shared__ uint4 s8_lds[];
-    char* const ring0 = reinterpret_cast<char*>(s8_lds) + 16;   // a pixel before the rings and one after
+    char* const ring0 = reinterpret_cast<char*>(s8_lds) + 16;   // s8_lds_bytes
     char* const img = reinterpret_cast<char*>(s8_lds) + c.n * kSRingBytes + 32;
     const int t = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
     const int ty = t / gridDim.x, tx = t - ty * gridDim.x;
@@ -318,7 +333,7 @@ __global__ __launch_bounds__(64 * kS8MaxWaves, 6) void acnet8_stream16(const Chu
         if (edge) strip_layer<Mma<T16>, Block8<T16>, true>(op, l, c.W, xs, sr, nsteps, in, out, lane);
         else strip_layer<Mma<T16>, Block8<T16>, false>(op, l, c.W, xs, sr, nsteps, in, out, lane);
     } else if (role == kS8Last) {
-        if (kSCols - 2 * c.n > 64) s8_last<T16, TIN, TOUT, IMG, FINAL, 5>(c, xs, sr, nsteps, img, ring0, lane);
+        if (s8_segments(c.n) == 5) s8_last<T16, TIN, TOUT, IMG, FINAL, 5>(c, xs, sr, nsteps, img, ring0, lane);
         else s8_last<T16, TIN, TOUT, IMG, FINAL, 4>(c, xs, sr, nsteps, img, ring0, lane);
     } else {
         if constexpr (IMG) {
@@ -375,7 +390,7 @@ hipError_t s8_launch(Chunk8 c, int cus, hipStream_t stream)
     const int waves = s8_roles(IMG, FINAL, c.n, c.roles);
     if (waves > kS8MaxWaves) return hipErrorInvalidValue;
     const int out_cols = kSCols - 2 * c.n, strips = (c.W + out_cols - 1) / out_cols;
-    const unsigned lds = c.n * kSRingBytes + 32 + (IMG ? kSImgBytes : 0);
+    const unsigned lds = s8_lds_bytes(IMG, c.n);
     // workgroups per CU: 160 KB of LDS and six waves per SIMD
     const int per_cu = std::min(static_cast<int>(160 * 1024 / lds), 6 / ((waves + 3) / 4));
     c.rows = strip_rows(strips, c.H, c.n, cus, per_cu);

@@ -47,3 +47,25 @@ def test_failed_launch_is_reported(trace, command):
     for k in range(len(launches)):
         (rc, _), = trace([f"fail {k}", command])
         assert rc == -5, f"launch {k} of {len(launches)} failed unnoticed"
+
+
+RING, IMG = 6 * 80 * 16, 6 * 84 * 4   # LDS bytes of a layer's ring of six rows and of the source rows
+
+
+@pytest.mark.parametrize("blocks", range(1, 65))
+def test_acnet8_streamed_lds(trace, blocks):
+    """The 16-bit ACNet<8> launches own every LDS byte they read.  The rings start 16 bytes in; the last
+    layer of a launch of n reads 16-pixel segments whole, five of them below 8 layers and four from
+    there on: the last lane's patch ends at pixel n - 1 + 15 + 16 (segments - 1) + 2 of a row of 80."""
+    for precision in (1, 2):
+        (rc, launches), = trace([f"net8 {blocks} {precision} 1 300 200"])
+        assert rc == 0
+        done = 0
+        for k, (_, _, _, _, lds) in enumerate(launches):
+            take = -(-(blocks - done) // (len(launches) - k))
+            n, done = take + (k == len(launches) - 1), done + take
+            segments = 5 if 80 - 2 * n > 64 else 4
+            last_row = 16 + (n - 1) * RING + 5 * 80 * 16
+            assert last_row + (n - 1 + 15 + 16 * (segments - 1) + 2 + 1) * 16 <= lds, (k, n)
+            assert 16 + n * RING + 16 + (IMG if k == 0 else 0) <= lds, (k, n)
+        assert done == blocks
