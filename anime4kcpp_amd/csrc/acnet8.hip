@@ -198,8 +198,8 @@ static void batch_launch(const SplitDesc* desc, int n, int total, const BatchSpl
     c.rows = sp.rows;
     for (int i = 0; i < NL; i++) c.la[i] = legacy_layer(first + i, wts, wa4, nullptr, 0);
     // the first launch writes map 0 (it reads no map), then 0 -> 1 -> 0 -> the outputs
-    hipLaunchKernelGGL((conv8_rows_batch<HEAD, NL, kRelu, MODE, TIN, TOUT>), dim3(total), dim3(rows8_threads<HEAD, NL>()), 0, stream,
-                       desc, n, total, sp.cols, ((first - 1) / NL & 1) == 0, c);
+    constexpr int threads = rows8_threads<HEAD, NL>();
+    hipLaunchKernelGGL((conv8_rows_batch<HEAD, NL, kRelu, MODE, TIN, TOUT>), strip_grid(total, 1, threads), dim3(threads), 0, stream, desc, n, total, sp.cols, ((first - 1) / NL & 1) == 0, c);
 }
 
 template <typename TIN, typename TOUT>

@@ -60,7 +60,7 @@ struct Chunk8 {
     const uint4* fin;       // 16-bit map in (no image head)
     uint4* fout;            // 16-bit map out (no final layer)
     long ss, ds, fp;
-    int W, H, rows;
+    int W, H, rows, strips;
     int l0;                 // block of this launch's layer 1
     int n;                  // layers after layer 0
     unsigned long long roles[2];   // S8Role of every wave, a byte each
@@ -313,8 +313,7 @@ __global__ __launch_bounds__(64 * kS8MaxWaves, 6) void acnet8_stream16(const Chu
     extern __shared__ uint4 s8_lds[];
     char* const ring0 = reinterpret_cast<char*>(s8_lds) + 16;   // s8_lds_bytes
     char* const img = reinterpret_cast<char*>(s8_lds) + c.n * kSRingBytes + 32;
-    const int t = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-    const int ty = t / gridDim.x, tx = t - ty * gridDim.x;
+    const int t = xcd_tile(strip_block(), gridDim.x * gridDim.y), ty = t / c.strips, tx = t - ty * c.strips;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const StripRows sr(ty * c.rows, min((ty + 1) * c.rows, c.H), c.H, c.n, IMG ? 1 : 0);
     const int nsteps = sr.steps(), xs = tx * (kSCols - 2 * c.n) - c.n;
@@ -389,12 +388,13 @@ hipError_t s8_launch(Chunk8 c, int cus, hipStream_t stream)
 {
     const int waves = s8_roles(IMG, FINAL, c.n, c.roles);
     if (waves > kS8MaxWaves) return hipErrorInvalidValue;
-    const int out_cols = kSCols - 2 * c.n, strips = (c.W + out_cols - 1) / out_cols;
+    const int out_cols = kSCols - 2 * c.n;
+    c.strips = (c.W + out_cols - 1) / out_cols;
     const unsigned lds = s8_lds_bytes(IMG, c.n);
     // workgroups per CU: 160 KB of LDS and six waves per SIMD
     const int per_cu = std::min(static_cast<int>(160 * 1024 / lds), 6 / ((waves + 3) / 4));
-    c.rows = strip_rows(strips, c.H, c.n, cus, per_cu);
-    hipLaunchKernelGGL((acnet8_stream16<T16, TIN, TOUT, IMG, FINAL>), dim3(strips, (c.H + c.rows - 1) / c.rows),
+    c.rows = strip_rows(c.strips, c.H, c.n, cus, per_cu);
+    hipLaunchKernelGGL((acnet8_stream16<T16, TIN, TOUT, IMG, FINAL>), strip_grid(c.strips, (c.H + c.rows - 1) / c.rows, 64 * waves),
                        dim3(64 * waves), lds, stream, c);
     return hipGetLastError();
 }

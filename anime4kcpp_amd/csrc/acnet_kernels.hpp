@@ -55,6 +55,16 @@ __device__ inline int xcd_tile(int b, int T)
     return x < r ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
 }
 
+// The grid of strips x segs workgroups of a strip kernel.  A dimension of a grid holds fewer than 2^32
+// threads, so the strips of an image too wide for that (358 Mpix at 768 threads and 64 columns) go along
+// y; strip_block() numbers the workgroups in either form, and a kernel counts its strips from the width.
+inline dim3 strip_grid(long strips, long segs, int threads)
+{
+    const unsigned a = static_cast<unsigned>(strips), b = static_cast<unsigned>(segs);
+    return strips * threads < 1L << 32 ? dim3(a, b) : dim3(b, a);
+}
+__device__ inline int strip_block() { return blockIdx.y * gridDim.x + blockIdx.x; }
+
 // Workgroups of a persistent launch: resident workgroups per CU x CUs, at most `tiles`, and
 // at most max_wg when max_wg > 0 (leaves CUs to work on other streams).
 int persistent_grid(const void* kernel, int threads, int tiles, int max_wg);

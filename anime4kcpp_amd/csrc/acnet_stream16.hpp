@@ -214,8 +214,8 @@ __global__ __launch_bounds__(kSLThreads, 6) void acnet_stream16(const void* __re
                                                                 const float* __restrict__ wa0, int rows)
 {
     __shared__ uint4 lds[kSLLds / 16];
-    const int t = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-    const int ty = t / gridDim.x, tx = t - ty * gridDim.x;
+    const int t = xcd_tile(strip_block(), gridDim.x * gridDim.y);
+    const int strips = (W + kSLOut - 1) / kSLOut, ty = t / strips, tx = t - ty * strips;
     legacy_strip<T16, TIN, TOUT>(src, ss, W, H, dst, ds, wts, wa, wa0, tx * kSLOut, ty * rows, min((ty + 1) * rows, H),
                                  reinterpret_cast<char*>(lds));
 }
@@ -260,7 +260,7 @@ static hipError_t launch_one(int cfg, const void* src, long ss, int W, int H, vo
 {
     const int strips = (W + kSLOut - 1) / kSLOut;
     const int rows = cfg ? kStreamConfigs[cfg].th : strip_rows(strips, H, kSLLayers, cus, 2);
-    hipLaunchKernelGGL((acnet_stream16<T16, TIN, TOUT>), dim3(strips, (H + rows - 1) / rows), dim3(kSLThreads), 0, stream,
+    hipLaunchKernelGGL((acnet_stream16<T16, TIN, TOUT>), strip_grid(strips, (H + rows - 1) / rows, kSLThreads), dim3(kSLThreads), 0, stream,
                        src, ss, W, H, dst, ds, wts, wa, wa0, rows);
     return hipGetLastError();
 }

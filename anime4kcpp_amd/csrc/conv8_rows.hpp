@@ -482,9 +482,10 @@ template <int HEAD, int NL, int MID, int MODE, typename TIN, typename TOUT>
 __global__ __launch_bounds__((rows8_threads<HEAD, NL>()), (rows8_waves<HEAD, NL>())) void conv8_rows(const Rows8 c)
 {
     __shared__ float4 lds[rows8_lds<HEAD, NL>() / 16];
-    const int t = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-    const int ty = t / gridDim.x, tx = t - ty * gridDim.x;
-    rows8_strip<HEAD, NL, MID, MODE, TIN, TOUT>(c, c.la, c.la[NL - 1], tx * (rows8_out<HEAD, NL>()), rows8_out<HEAD, NL>(), ty * c.rows,
+    constexpr int out = rows8_out<HEAD, NL>();
+    const int t = xcd_tile(strip_block(), gridDim.x * gridDim.y);
+    const int strips = (c.W + out - 1) / out, ty = t / strips, tx = t - ty * strips;
+    rows8_strip<HEAD, NL, MID, MODE, TIN, TOUT>(c, c.la, c.la[NL - 1], tx * out, out, ty * c.rows,
                                                 min((ty + 1) * c.rows, c.H), (tx + ty) % NL, reinterpret_cast<char*>(lds));
 }
 
@@ -495,7 +496,7 @@ __global__ __launch_bounds__((rows8_threads<HEAD, NL>()), (rows8_waves<HEAD, NL>
                                                                                   int out, int from_m1, const Rows8 c0)
 {
     __shared__ float4 lds[rows8_lds<HEAD, NL>() / 16];
-    const int t = xcd_tile(blockIdx.x, total);
+    const int t = xcd_tile(strip_block(), total);
     const SplitDesc d = find_tile(desc, n, t);
     const int local = t - d.first_tile, ty = local / d.tiles_x, tx = local - ty * d.tiles_x;
     RowsIo c = c0;
@@ -556,8 +557,9 @@ inline hipError_t launch_rows8(Rows8 c, int cus, hipStream_t stream)
 {
     const int out = rows8_out<HEAD, NL>(), strips = (c.W + out - 1) / out;
     c.rows = rows8_rows(strips, c.H, NL, HEAD == kRowsMap ? 0 : 1, cus, rows8_per_cu<HEAD, NL>());
-    const dim3 grid(strips, (c.H + c.rows - 1) / c.rows), block(rows8_threads<HEAD, NL>());
-    hipLaunchKernelGGL((conv8_rows<HEAD, NL, MID, MODE, TIN, TOUT>), grid, block, 0, stream, c);
+    constexpr int threads = rows8_threads<HEAD, NL>();
+    hipLaunchKernelGGL((conv8_rows<HEAD, NL, MID, MODE, TIN, TOUT>), strip_grid(strips, (c.H + c.rows - 1) / c.rows, threads),
+                       dim3(threads), 0, stream, c);
     return hipGetLastError();
 }
 

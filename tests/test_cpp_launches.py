@@ -69,3 +69,16 @@ def test_acnet8_streamed_lds(trace, blocks):
             assert last_row + (n - 1 + 15 + 16 * (segments - 1) + 2 + 1) * 16 <= lds, (k, n)
             assert 16 + n * RING + 16 + (IMG if k == 0 else 0) <= lds, (k, n)
         assert done == blocks
+
+
+WIDE = [f"{c} {w} {h}" for w, h in [(360000000, 1), (400000000, 2), (1 << 29, 1)]
+        for c in ["net8 8 1 1", "net8 18 2 1", "net8 64 1 1", "net8 4 0 1", "net8 8 0 1", "net8 18 0 516"]]
+WIDE += ["legacy 1 -1 1 360000000 1", "legacy 2 0 516 500000000 1", "layers 1 536870912 1", "batch_layers 3 268435456 1"]
+
+
+@pytest.mark.parametrize("command", WIDE)
+def test_very_wide_images(trace, command):
+    """Images of more columns than 2^32 threads make in strips: accepted, in a grid whose dimensions each
+    hold fewer than 2^32 threads (the stand-in refuses others, as the runtime does)."""
+    (rc, launches), = trace([command])
+    assert rc == 0 and launches

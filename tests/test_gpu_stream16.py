@@ -105,3 +105,16 @@ def test_acnet8_crop(cuda, blocks):
     torch.cuda.synchronize()
     assert torch.equal(part[2 * m:2 * (h - m), 2 * m:2 * (w - m)], whole[2 * (y + m):2 * (y + h - m), 2 * (x + m):2 * (x + w - m)])
     net.close()
+
+
+def test_more_columns_than_one_grid_dimension(net, cuda):
+    """360 million columns, a row high: the strips go along the grid's y.  Around the image's ends and at
+    spots between (a strip's first and last columns), the outputs are those of a part of the image."""
+    w = 360_000_001
+    src = torch.from_numpy(synth.flat_shaded(43, 1 << 16, 1, dtype=np.uint8)).to(cuda).repeat(1, w // (1 << 16) + 1)[:, :w].contiguous()
+    got = net.upscale(src, precision="fp16")
+    for x in (0, 64 * 1234567 - 200, w // 2, w - 400):
+        a, b = max(x - 20, 0), min(x + 420, w)
+        part = net.upscale(src[:, a:b].contiguous(), precision="fp16")
+        lo, hi = (0 if a == 0 else x), (w if b == w else x + 400)
+        assert torch.equal(got[:, 2 * lo:2 * hi], part[:, 2 * (lo - a):2 * (hi - a)]), x
