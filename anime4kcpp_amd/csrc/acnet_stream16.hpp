@@ -220,7 +220,10 @@ __global__ __launch_bounds__(kSLThreads, 6) void acnet_stream16(const void* __re
                                  reinterpret_cast<char*>(lds));
 }
 
-// Persistent batched form: resident workgroups take strips of `rows` rows from a queue.
+// Persistent batched form: resident workgroups (at most one per strip) take strips of `rows` rows, the
+// first one by their own number and the rest from a queue.  Drawing the first ones too let the workgroups
+// that started first take a second strip before the last ones had drawn any, which then found the queue
+// empty (150 strips of 20 rows: 39.5 us against 23.8 now; three u8 images of 700 x 500 in FP16: 72 against 48).
 template <typename T16, typename TIN, typename TOUT>
 __global__ __launch_bounds__(kSLThreads, 6) void acnet_stream16_batch(const BatchDesc* __restrict__ desc, int n, int total,
                                                                       int* __restrict__ counter,
@@ -230,14 +233,12 @@ __global__ __launch_bounds__(kSLThreads, 6) void acnet_stream16_batch(const Batc
 {
     __shared__ uint4 lds[kSLLds / 16];
     __shared__ int s_tile;
-    if (threadIdx.x == 0) s_tile = atomicAdd(counter, 1);
-    __syncthreads();
-    int t = __builtin_amdgcn_readfirstlane(s_tile);   // uniform: keeps the strip's state scalar
+    int t = blockIdx.x;
     while (t < total) {
         // The next strip is drawn as this one starts and read once it is done, so the atomic's
         // round trip overlaps the strip.  Each workgroup draws exactly one index past its last.
         int next = 0;
-        if (threadIdx.x == 0) next = atomicAdd(counter, 1);
+        if (threadIdx.x == 0) next = gridDim.x + atomicAdd(counter, 1);
         const BatchDesc d = find_tile(desc, n, t);
         const int local = t - d.first_tile;
         const int ly = local / d.tiles_x;

@@ -118,3 +118,23 @@ def test_more_columns_than_one_grid_dimension(net, cuda):
         part = net.upscale(src[:, a:b].contiguous(), precision="fp16")
         lo, hi = (0 if a == 0 else x), (w if b == w else x + 400)
         assert torch.equal(got[:, 2 * lo:2 * hi], part[:, 2 * (lo - a):2 * (hi - a)]), x
+
+
+def test_batch_strips_start_together(net, cuda):
+    """200 strips of 128 rows on 256 compute units take about as long as 16 of them: every workgroup of
+    the queue has one strip before any takes a second (which makes it twice as long)."""
+    def us(w):
+        src = [torch.zeros((128, w), dtype=torch.uint8, device=cuda)]
+        dst = [torch.empty((256, 2 * w), dtype=torch.uint8, device=cuda)]
+        best = float("inf")
+        for _ in range(8):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(10):
+                net.upscale_batch(src, dst, precision="fp16", config=1)
+            e1.record()
+            torch.cuda.synchronize()
+            best = min(best, e0.elapsed_time(e1) * 100)
+        return best
+    few, many = us(16 * 64), us(200 * 64)
+    assert many < 1.5 * few, (few, many)
