@@ -3,7 +3,8 @@
 // over libamdhip64's for libac_hip.so, so no device is needed and none is used.
 //
 // Commands, one a line on stdin; every answer is a line "rc <code> <seconds>", then one line per launch,
-// "<kernel> <grid x> <grid y> <block x> <LDS bytes>", then "end":
+// "<kernel> <grid x> <grid y> <block x> <LDS bytes> <strips> <rows>", then "end" (strips and rows of a
+// strip: of the batch kernels that take them as arguments, else 0):
 //   legacy <precision> <config> <type> <w> <h>      achip_pass_config (config -1: ACHIP_AUTO)
 //   layers <type> <w> <h>                           achip_pass_layers
 //   net8 <blocks> <precision> <type> <w> <h>        achip_pass8_precision
@@ -11,6 +12,8 @@
 //   fsr <channels> <blocks> <type> <w> <h>          achip_pass_net
 //   batch <precision> <config> <n> <w> <h>          achip_pass_batch, u8, n images of w x h
 //   batch_layers <n> <w> <h>                        achip_pass_batch_layers, the same
+//   images <precision> <w> <h> <w> <h> ...          achip_pass_batch, u8, images of these sizes
+//   images_layers <w> <h> <w> <h> ...               achip_pass_batch_layers, the same
 //   tune <precision> <w> <h> <us of each configuration>   achip_autotune, u8, with these times
 //   fail <k>                                        launch k (from 0) of the next command fails
 #ifndef __HIP_PLATFORM_AMD__
@@ -36,6 +39,7 @@ struct Launch {
     std::string name;
     dim3 grid, block;
     size_t lds;
+    int strips, rows;
 };
 
 std::map<const void*, std::string>& names()
@@ -91,9 +95,13 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
     *stream = nullptr;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void**, size_t lds, hipStream_t)
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t)
 {
-    launches.push_back({ names()[f], grid, block, lds });
+    const std::string& name = names()[f];
+    const bool queue = name.find("acnet_stream16_batch") != std::string::npos;   // desc, n, total, counter, 3 weights, rows
+    const bool layers = name.find("conv8_rows_batch") != std::string::npos;      // desc, n, total, ...
+    launches.push_back({ name, grid, block, lds, queue || layers ? *static_cast<int*>(args[2]) : 0,
+                         queue ? *static_cast<int*>(args[7]) : 0 });
     const bool empty = !grid.x || !grid.y || !grid.z || !block.x;
     // a dimension of the grid holds fewer than 2^32 threads, a workgroup at most 1024, a CU 160 KB of LDS
     const bool large = uint64_t(grid.x) * block.x > UINT32_MAX || uint64_t(grid.y) * block.y > UINT32_MAX || block.x > 1024 ||
@@ -200,20 +208,23 @@ int run(const std::string& what, std::istringstream& in)
         const Image im(type, w, h);
         const size_t need = achip_net_workspace_bytes(net, w, h);
         rc = achip_pass_net(net, im.src, im.ss, type, w, h, im.dst, im.ds, type, reinterpret_cast<void*>(allocate(need)), need, nullptr);
-    } else if (what == "batch" || what == "batch_layers") {
+    } else if (what == "batch" || what == "batch_layers" || what == "images" || what == "images_layers") {
+        const bool queue = what == "batch" || what == "images", same = what == "batch" || what == "batch_layers";
         int precision = 0, config = 0, n = 0;
-        if (what == "batch") in >> precision >> config;
-        in >> n >> w >> h;
+        if (queue) in >> precision;
+        if (what == "batch") in >> config;
+        if (same) in >> n >> w >> h;
         if (achip_net_create(0, z, z, &net)) return -1000;
         std::vector<ACHipImage> images;
-        for (int i = 0; i < n; i++) {
+        while (same ? static_cast<int>(images.size()) < n : static_cast<bool>(in >> w >> h)) {
             const Image im(type, w, h);
             images.push_back({ im.src, im.ss, im.dst, im.ds, w, h });
         }
-        const size_t need = what == "batch" ? achip_batch_workspace_bytes(n) : achip_pass_batch_layers_bytes(images.data(), n);
+        n = static_cast<int>(images.size());
+        const size_t need = queue ? achip_batch_workspace_bytes(n) : achip_pass_batch_layers_bytes(images.data(), n);
         void* ws = reinterpret_cast<void*>(allocate(need));
-        rc = what == "batch" ? achip_pass_batch(net, precision, config, type, type, images.data(), n, ws, need, nullptr)
-                             : achip_pass_batch_layers(net, type, type, images.data(), n, ws, need, nullptr);
+        rc = queue ? achip_pass_batch(net, precision, config, type, type, images.data(), n, ws, need, nullptr)
+                   : achip_pass_batch_layers(net, type, type, images.data(), n, ws, need, nullptr);
     } else if (what == "tune") {
         int precision = 0, best = 0;
         in >> precision >> w >> h;
@@ -251,7 +262,7 @@ int main()
         memory.clear();
         std::printf("rc %d %.6f\n", rc, s);
         for (const Launch& l : launches)
-            std::printf("%s %u %u %u %zu\n", l.name.c_str(), l.grid.x, l.grid.y, l.block.x, l.lds);
+            std::printf("%s %u %u %u %zu %d %d\n", l.name.c_str(), l.grid.x, l.grid.y, l.block.x, l.lds, l.strips, l.rows);
         std::printf("end\n");
     }
     return 0;

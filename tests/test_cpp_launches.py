@@ -13,7 +13,7 @@ ROOT = os.path.dirname(HERE)
 
 @pytest.fixture(scope="module")
 def trace(tmp_path_factory):
-    """trace(commands): [(return code, [(kernel, grid x, grid y, block x, LDS bytes), ...]), ...]"""
+    """trace(commands): [(return code, [(kernel, grid x, grid y, block x, LDS bytes, strips, rows), ...]), ...]"""
     exe = str(tmp_path_factory.mktemp("trace") / "launch_trace")
     libdir = os.path.dirname(_native.LIB_PATH)
     subprocess.run(["g++", "-std=c++17", "-O1", "-rdynamic", "-I" + os.path.join(ROOT, "include"), "-I/opt/rocm/include",
@@ -61,7 +61,7 @@ def test_acnet8_streamed_lds(trace, blocks):
         (rc, launches), = trace([f"net8 {blocks} {precision} 1 300 200"])
         assert rc == 0
         done = 0
-        for k, (_, _, _, _, lds) in enumerate(launches):
+        for k, (_, _, _, _, lds, _, _) in enumerate(launches):
             take = -(-(blocks - done) // (len(launches) - k))
             n, done = take + (k == len(launches) - 1), done + take
             segments = 5 if 80 - 2 * n > 64 else 4
@@ -82,3 +82,28 @@ def test_very_wide_images(trace, command):
     hold fewer than 2^32 threads (the stand-in refuses others, as the runtime does)."""
     (rc, launches), = trace([command])
     assert rc == 0 and launches
+
+
+# Batches of u8 images (widths and heights in turn) and the us of one FP16 launch on an MI355X at heights of
+# strips from 8 to 256 rows
+BATCHES16 = [
+    (
+     "762 341 276 621 296 442 967 942 294 278 345 880 255 347 289 298 550 325 461 760 748 465 ",
+     {8: 188, 12: 151, 16: 133, 20: 123, 24: 116, 32: 109, 40: 112, 48: 103, 64: 107, 80: 112, 96: 118, 128: 104, 192: 123, 256: 122}),
+    (
+     "474 265 148 84 1478 655 122 384 562 1088 135 151 99 378 1144 613 84 183 68 91 274 88 131 119 217 918 116 409 201 140 ",
+     {8: 184, 12: 148, 16: 132, 20: 121, 24: 114, 32: 105, 40: 109, 48: 97, 64: 105, 80: 110, 96: 117, 128: 105, 192: 139, 256: 122}),
+    (
+     "36 174 69 468 430 83 202 148 79 123 110 136 577 299 38 97 605 327 206 232 260 55 114 78 60 264 38 58 281 485 84 429 404 "
+     "54 516 56 138 44 45 245 413 47 90 209 199 51 268 47 545 247 244 529 69 62 219 486 542 361 204 99 354 225 463 322 146 233 ",
+     {8: 132, 12: 108, 16: 97, 20: 94, 24: 88, 32: 85, 40: 84, 48: 87, 64: 90, 80: 76, 96: 83, 128: 99, 192: 95, 256: 118}),
+]
+
+
+@pytest.mark.parametrize("sizes,us", BATCHES16, ids=["11", "15", "33"])
+def test_batch_strip_height(trace, sizes, us):
+    """The height that the 16-bit batch takes for its strips is, by the measured times, within 12% of the
+    best one (the times of one height differ by up to 4% from run to run)."""
+    (rc, launches), = trace(["images 1 " + sizes])
+    assert rc == 0
+    assert us[launches[0][6]] <= 1.12 * min(us.values()), launches[0][6]
