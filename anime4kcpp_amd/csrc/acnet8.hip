@@ -157,14 +157,16 @@ static hipError_t legacy_split_t(const void* src, long ss, int W, int H, void* d
 
 // What a launch of n strips of `rows` rows takes: a strip has two steps per layer after the first and
 // about three to start, a step takes a fixed part and one for every layer and strip on the CU, and
-// strips beyond one round of the CUs come in where others end, half a round late at the end.
-// Measured, layers per launch / rows: 300 x 143 .. 483 x 409, four images, 2 / 12 88 us, 2 / 20 98,
-// 4 / 20 88, 4 / 40 92 (62 x 16 tiles before: 91); eight of 250 x 200 2 / 8 81, 2 / 20 97, 4 / 18 83,
-// 4 / 40 93; four of 512 x 512 2 / 20 148, 2 / 32 173, 4 / 28 159 (before: 183).
+// strips beyond one round of the CUs come in where others end, a third of a round late at the end.
+// One round alone takes a fifth more: its strips are not spread evenly over the CUs, and a short
+// image's strips hold their places for a whole strip's steps.
+// Over 28 batches (u8) within 1.4% of the best of 12 heights and both numbers of layers on average, 8%
+// at worst; without the fifth 3.6% and 33%: 48 of 300 x 200 in strips of 64 rows 430 us, 40 rows 322
+// (62 x 16 tiles before: 453), 24 of 5.2 Mpix 4 / 256 790, 2 / 48 643 (before: 760).
 static double batch_cost(double n, int rows, int layers, int per_cu, int cus)
 {
     const double at = std::min<double>(per_cu, std::ceil(n / cus)), rounds = n / (at * cus);
-    return (rows / 2 + 2 * (layers - 1) + 3) * (4.0 + at * layers) * (rounds <= 1.0 ? 1.0 : rounds + 0.5);
+    return (rows / 2 + 2 * (layers - 1) + 3) * (4.0 + at * layers) * (rounds <= 1.0 ? 1.2 : rounds + 0.3);
 }
 
 BatchSplit legacy_batch_split(const SplitDesc* desc, int n, int cus)

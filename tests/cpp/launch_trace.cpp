@@ -99,9 +99,11 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
 {
     const std::string& name = names()[f];
     const bool queue = name.find("acnet_stream16_batch") != std::string::npos;   // desc, n, total, counter, 3 weights, rows
-    const bool layers = name.find("conv8_rows_batch") != std::string::npos;      // desc, n, total, ...
+    const bool layers = name.find("conv8_rows_batch") != std::string::npos;      // desc, n, total, out, from_m1, Rows8
     launches.push_back({ name, grid, block, lds, queue || layers ? *static_cast<int*>(args[2]) : 0,
-                         queue ? *static_cast<int*>(args[7]) : 0 });
+                         queue    ? *static_cast<int*>(args[7])
+                         : layers ? *reinterpret_cast<int*>(static_cast<char*>(args[5]) + 64)   // after 7 pointers and longs, W, H
+                                  : 0 });
     const bool empty = !grid.x || !grid.y || !grid.z || !block.x;
     // a dimension of the grid holds fewer than 2^32 threads, a workgroup at most 1024, a CU 160 KB of LDS
     const bool large = uint64_t(grid.x) * block.x > UINT32_MAX || uint64_t(grid.y) * block.y > UINT32_MAX || block.x > 1024 ||

@@ -107,3 +107,31 @@ def test_batch_strip_height(trace, sizes, us):
     (rc, launches), = trace(["images 1 " + sizes])
     assert rc == 0
     assert us[launches[0][6]] <= 1.12 * min(us.values()), launches[0][6]
+
+
+# The same for achip_pass_batch_layers, by (layers per launch, rows)
+BATCHES32 = [
+    ("300 200 " * 48,
+     {(2, 8): 406, (2, 12): 376, (2, 16): 372, (2, 20): 353, (2, 24): 371, (2, 28): 371, (2, 32): 390, (2, 40): 322, (2, 48): 373, (2, 64): 393, (2, 96): 453,
+      (4, 8): 581, (4, 12): 500, (4, 16): 465, (4, 20): 439, (4, 24): 435, (4, 28): 438, (4, 32): 428, (4, 40): 410, (4, 48): 440, (4, 64): 491, (4, 96): 494}),
+    (
+     "339 399 732 849 242 307 977 285 667 398 657 927 594 439 394 632 639 452 495 553 356 314 582 277 609 842 878 352 456 1021 "
+     "411 1138 324 896 252 680 847 563 644 1006 1146 314 541 251 430 297 304 636 270 301 240 858 347 265 632 737 642 562 551 "
+     "739 386 898 709 921 969 894 538 540 ",
+     {(2, 8): 1532, (2, 12): 1392, (2, 16): 1360, (2, 20): 1336, (2, 24): 1319, (2, 28): 1296, (2, 32): 1279, (2, 40): 1292, (2, 48): 1268, (2, 64): 1260, (2, 96): 1300,
+      (4, 8): 2076, (4, 12): 1756, (4, 16): 1604, (4, 20): 1512, (4, 24): 1441, (4, 28): 1409, (4, 32): 1383, (4, 40): 1345, (4, 48): 1320, (4, 64): 1315, (4, 96): 1331}),
+    (
+     "467 599 669 909 596 871 136 337 910 494 833 162 339 214 397 422 132 201 229 861 629 178 672 171 462 167 128 784 198 200 "
+     "987 785 234 945 393 524 196 906 538 955 821 238 271 181 173 147 240 449 ",
+     {(2, 8): 735, (2, 12): 685, (2, 16): 669, (2, 20): 657, (2, 24): 649, (2, 28): 639, (2, 32): 634, (2, 40): 642, (2, 48): 643, (2, 64): 675, (2, 96): 689,
+      (4, 8): 992, (4, 12): 843, (4, 16): 772, (4, 20): 729, (4, 24): 706, (4, 28): 696, (4, 32): 685, (4, 40): 678, (4, 48): 677, (4, 64): 676, (4, 96): 725}),
+]
+
+
+@pytest.mark.parametrize("sizes,us", BATCHES32, ids=["48", "34", "24"])
+def test_batch_layers_strips(trace, sizes, us):
+    """Layers per launch and heights: within 10% of the best measured."""
+    (rc, launches), = trace(["images_layers " + sizes])
+    assert rc == 0
+    cut = 8 // len(launches), launches[0][6]
+    assert us[cut] <= 1.1 * min(us.values()), cut
