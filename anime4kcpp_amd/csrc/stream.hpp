@@ -119,11 +119,13 @@ __device__ __forceinline__ void strip_loader(const void* __restrict__ src, long 
 inline int strip_steps(int rows, int layers) { return (rows + 1) / 2 + kSLag * (layers + 1); }
 
 // Rows per strip of an image of `strips` strips x H rows on a device of `cus` compute units that
-// hold per_cu workgroups each.  Measured on 1080p and 4K u8 in FP16 (8 layers, two per CU): a
-// step takes about 0.72 us with one workgroup per CU and 0.97 us with two, so the candidates are
-// the heights that fill one workgroup per CU or 1, 2, 4 rounds of all, and the cheapest by
-// that count is taken.  1080p: 64 rows 46 us (32: 56, 136: 62); 4K: 270 rows 150 (128: 149, 64:
-// 163); 256 x 256: 4 rows 12.4 (2: 14.5, 16: 17).
+// hold per_cu workgroups each.  Measured (u8 in FP16, 4 to 18 blocks and ACNetLegacy, 256 x 256 to 4K): a
+// strip of r rows with a compute unit of its own takes time with r + 3 (layers + 1) (the steps that
+// fill and drain it, two per layer, run fewer layers than the rest), two to a compute unit 4/3 of that.
+// So the candidates are the heights that fill one workgroup per CU or 1, 2, 4 rounds of all, and the
+// cheapest by that count is taken.  ACNetLegacy, us: 1080p 64 rows 47 (36: 58, 80: 55); 4K 270 rows 150
+// (128: 149, 64: 163); 800 x 600 16 rows 21.8 (32 rows, one per CU: 23.7; 64 x 32 tiles before: 23.1);
+// 256 x 256 4 rows 12.7 (8: 13.8, 16: 17).
 inline int strip_rows(long strips, int H, int layers, int cus, int per_cu)
 {
     long best = -1;
@@ -135,7 +137,7 @@ inline int strip_rows(long strips, int H, int layers, int cus, int per_cu)
         if (segs < 1) continue;
         const int r = static_cast<int>(((H + segs - 1) / segs + 1) / 2 * 2);
         const long n = strips * ((H + r - 1) / r);
-        const long cost = strip_steps(r, layers) * (n <= cus ? 3L : (2L + per_cu) * ((n + all - 1) / all));
+        const long cost = (r + 3L * (layers + 1)) * (n <= cus ? 3L : (2L + per_cu) * ((n + all - 1) / all));
         if (best < 0 || cost < best) {
             best = cost;
             rows = r;

@@ -135,3 +135,22 @@ def test_batch_layers_strips(trace, sizes, us):
     assert rc == 0
     cut = 8 // len(launches), launches[0][6]
     assert us[cut] <= 1.1 * min(us.values()), cut
+
+
+# u8 passes and their us by the height of strips, in the launches that are named (the second and third of
+# FSRCNNX<8>: its two-layer ones)
+HEIGHTS16 = [("legacy 1 -1 1 800 600", 0, {16: 21.8, 18: 22.4, 20: 23.0, 22: 24.2, 32: 23.7}),
+             ("legacy 1 -1 1 960 540", 0, {16: 21.6, 18: 22.2, 20: 23.0, 32: 23.7, 36: 25.1}),
+             ("legacy 2 -1 1 644 716", 0, {16: 22.5, 18: 23.3, 20: 24.3, 32: 23.7, 36: 25.1}),
+             ("legacy 1 -1 1 1920 1080", 0, {36: 58.0, 48: 59.9, 64: 46.9, 72: 50.2, 80: 54.7}),
+             ("net8 8 1 1 800 600", 0, {16: 33.5, 18: 34.8, 20: 36.4, 32: 33.8, 36: 35.6})]
+
+
+@pytest.mark.parametrize("command,launch,us", HEIGHTS16)
+def test_strip_height(trace, command, launch, us):
+    """The height of a pass's strips is, by the measured times, within 4% of the best one."""
+    (rc, launches), = trace([command])
+    assert rc == 0
+    h = int(command.split()[-1])
+    got = [t for r, t in us.items() if -(-h // r) == launches[launch][2]]
+    assert got and min(got) <= 1.04 * min(us.values()), launches[launch]
