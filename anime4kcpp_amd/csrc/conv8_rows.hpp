@@ -529,12 +529,16 @@ inline Rows8 rows8_args(const float4* in, float4* out, long fp, int W, int H, st
     return c;
 }
 
-// Rows per strip.  A strip of r rows takes r / 2 + 2 (layers - 1) steps and about two more to
+// Rows per strip.  A strip of r rows takes r / 2 + 2 (layers - 1) steps and one or two more to
 // start; with w waves per SIMD at work a step takes about 1150 (1 + w) cycles (two layers at
 // 1080p: one strip per CU 2280, two 3510, three 4640, four 5660), so the heights that put 1, 2, ..
-// strips on every CU are compared by that, and several rounds of the last.
+// strips on every CU are compared by that, and several rounds of the last.  One step to start for one
+// or two layers, by small images: FSRCNNX<8> 640 x 360 43.8 us with two (16 rows, one strip per CU), 40.0
+// with one (8 rows, two; 64 x 16 tiles before: 42.7), 327 x 641 44.4 / 39.7 (41.8); ACNetLegacy and
+// ACNet<8> within 2% either way.
 inline int rows8_rows(long strips, int H, int layers, int lead, int cus, int per_cu)
 {
+    const int start = layers <= 2 ? 1 : 2;
     long best = -1;
     int rows = (H + 1) / 2 * 2;
     for (int k = 1; k <= per_cu + 2; k++) {
@@ -543,7 +547,7 @@ inline int rows8_rows(long strips, int H, int layers, int lead, int cus, int per
         if (segs < 1) continue;
         const int r = static_cast<int>(((H + segs - 1) / segs + 1) / 2 * 2);
         const long n = strips * ((H + r - 1) / r);
-        const long cost = (r / 2 + 2 * (layers - 1 + lead) + 2) * (2L + at * layers) * ((n + static_cast<long>(at) * cus - 1) / (static_cast<long>(at) * cus));
+        const long cost = (r / 2 + 2 * (layers - 1 + lead) + start) * (2L + at * layers) * ((n + static_cast<long>(at) * cus - 1) / (static_cast<long>(at) * cus));
         if (best < 0 || cost < best) {
             best = cost;
             rows = r;
