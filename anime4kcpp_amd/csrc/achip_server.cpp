@@ -47,6 +47,7 @@ constexpr int kMaxStreams = 64;
 constexpr int kRing = 4;              // descriptor workspaces (steps in flight <= kRing - 2)
 constexpr int kMaxStepItems = 512;    // descriptors per step
 constexpr size_t kBlock = 2u << 20;   // allocation granularity
+constexpr long kStepTilePx = 64 * 32;   // ACHipServerConfig.step_tiles counts these
 
 double ms_between(Clock::time_point a, Clock::time_point b)
 {
@@ -526,7 +527,7 @@ bool ACHipServer::build_step()
     std::vector<achip::BatchDesc> d16;
     int n = 0;
     long total = 0, total16 = 0;
-    long budget = cfg.step_tiles;
+    long budget = cfg.step_tiles * kStepTilePx;
     std::vector<std::shared_ptr<Req>> finishing, members;
     for (const std::shared_ptr<Req>& q : active) {
         if (budget <= 0 || n + static_cast<int>(d16.size()) >= kMaxStepItems) break;
@@ -535,13 +536,14 @@ bool ACHipServer::build_step()
         const Plane& a = q->luma[q->pass];
         const Plane& b = q->luma[q->pass + 1];
         const int tiles_x = (a.w + tw - 1) / tw, tiles_y = (a.h + th - 1) / th;
-        const int rows = std::min<long>(tiles_y - q->next_row, std::max<long>(1, budget / tiles_x));
+        const long row_px = static_cast<long>(tiles_x) * tw * th;
+        const int rows = std::min<long>(tiles_y - q->next_row, std::max<long>(1, budget / row_px));
         long& tot = q->type == kU16 ? total16 : total;
         const achip::BatchDesc d{ a.ptr, b.ptr, a.stride, b.stride, a.w, a.h, tiles_x, static_cast<int>(tot), q->next_row };
         if (q->type == kU16) d16.push_back(d);
         else desc[n++] = d;
         tot += static_cast<long>(rows) * tiles_x;
-        budget -= static_cast<long>(rows) * tiles_x;
+        budget -= rows * row_px;
         q->next_row += rows;
         if (q->next_row == tiles_y) {
             q->pass++;
@@ -608,11 +610,11 @@ hipError_t ACHipServer::launch_finish(const Req& q)
 
 // A step of a layer-by-layer net: the admitted one-offs' next passes, each whole (its layer
 // launches in turn on the batch stream), in admission order until the step's pixel budget
-// (step_tiles x the tile area) is spent; then the finishing kernels of the requests whose
+// (step_tiles x kStepTilePx) is spent; then the finishing kernels of the requests whose
 // last pass this step ran.
 bool ACHipServer::build_layered_step(Step& step)
 {
-    long budget = static_cast<long>(cfg.step_tiles) * tw * th;
+    long budget = cfg.step_tiles * kStepTilePx;
     std::vector<std::shared_ptr<Req>> finishing, members;
     hipError_t e = hipSuccess;
     for (const std::shared_ptr<Req>& q : active) {
@@ -790,7 +792,7 @@ int achip_server_create(ACHipNet* net, const ACHipServerConfig* config, ACHipSer
     const bool layered = net->blocks || net->lfamily;
     if (net->lfamily && c.precision != ACHIP_FP32) return ACHIP_EINVAL;   // ArtCNN and FSRCNNX run in FP32 only
     if (c.hbm_budget == 0) c.hbm_budget = static_cast<size_t>(16) << 30;
-    if (c.step_tiles <= 0) c.step_tiles = c.precision == ACHIP_FP32 ? 2048 : 6144;   // 4.2 / 25.2 Mpix
+    if (c.step_tiles <= 0) c.step_tiles = c.precision == ACHIP_FP32 ? 2048 : 12288;   // 4.2 / 25.2 Mpix
     if (c.max_workgroups < 0) return ACHIP_EINVAL;
     auto s = std::make_unique<ACHipServer>();
     s->net = net;

@@ -309,7 +309,8 @@ typedef struct ACHipRequest {
 typedef struct ACHipServerConfig {
     int precision;          /* ACHIP_FP32 / FP16 / BF16 */
     size_t hbm_budget;      /* bytes of device memory for request buffers (0: 16 GiB) */
-    int step_tiles;         /* tile budget of one batched step (0: a default for the precision) */
+    int step_tiles;         /* budget of one batched step in tiles of 64 x 32 input pixels, whatever the
+                               precision's own tiles are (0: a default for the precision) */
     int max_workgroups;     /* grid cap of a batched step (0: a default that leaves CUs for frames) */
 } ACHipServerConfig;
 

@@ -261,3 +261,14 @@ def test_page_locked_planes_equal_pageable(net):
         for pa, pb in zip(a, b):
             assert np.array_equal(pa, pb), f"request {i}: page-locked planes differ from pageable ones"
     assert np.array_equal(outs[-1][0], want[first_rgb][0])
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp16", "bf16"])
+def test_step_budget_counts_64x32_tiles(net, prec):
+    """step_tiles is in tiles of 64 x 32 pixels in every precision: 64 x 1280 pixels are 40 of them, 20
+    steps of two."""
+    y = synth.flat_shaded(77, 64, 1280, dtype=np.uint8)
+    with hip.Server(net, prec, step_tiles=2) as srv:
+        out = np.empty((2560, 128), np.uint8)
+        srv.wait(srv.submit(hip.REQ_LUMA, [y], 2, -1, [out]), 60000)
+        assert srv.stats()["steps"] == 20
