@@ -93,6 +93,9 @@ extern const int kStreamConfigCount;
 hipError_t launch_stream16(int bf16, int cfg, int stype, int dtype, const void* src, long sstride, int W, int H,
                            void* dst, long dstride, const float* wts, const void* wa, const float* wa0, int cus,
                            hipStream_t stream);
+// Whether the fixed strip height of configuration cfg suits a w x h image: its cost by the rule for
+// heights is within 5% of the one that configuration 0 takes (true for configuration 0).
+bool stream16_config_suits(int cfg, int w, int h, int cus);
 // Rows per tile of a batch of n images (their sizes) under configuration cfg.
 int stream16_batch_rows(int cfg, const BatchDesc* desc, int n, int cus);
 

@@ -1,5 +1,7 @@
 // The FP16 kernels of the streamed ACNetLegacy pass (acnet_stream16.hpp), its configurations and
 // its launch entry points; the BF16 kernels are compiled beside it (acnet_stream16_bf16.hip).
+#include <algorithm>
+
 #include "acnet_stream16.hpp"
 
 namespace achip {
@@ -12,6 +14,14 @@ const Fp32Config kStreamConfigs[] = {
     { kSLOut, 128, kSLThreads, 0, static_cast<int>(kSLLds) },
 };
 const int kStreamConfigCount = sizeof(kStreamConfigs) / sizeof(kStreamConfigs[0]);
+
+bool stream16_config_suits(int cfg, int w, int h, int cus)
+{
+    if (cfg == 0) return true;
+    const long strips = (static_cast<long>(w) + kSLOut - 1) / kSLOut;
+    const long rule = strip_cost(strips, h, kSLLayers, cus, 2, strip_rows(strips, h, kSLLayers, cus, 2));
+    return strip_cost(strips, h, kSLLayers, cus, 2, std::min(kStreamConfigs[cfg].th, (h + 1) / 2 * 2)) * 20 <= rule * 21;
+}
 
 int stream16_batch_rows(int cfg, const BatchDesc* desc, int n, int cus)
 {

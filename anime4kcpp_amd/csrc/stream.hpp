@@ -126,6 +126,12 @@ inline int strip_steps(int rows, int layers) { return (rows + 1) / 2 + kSLag * (
 // cheapest by that count is taken.  ACNetLegacy, us: 1080p 64 rows 47 (36: 58, 80: 55); 4K 270 rows 150
 // (128: 149, 64: 163); 800 x 600 16 rows 21.8 (32 rows, one per CU: 23.7; 64 x 32 tiles before: 23.1);
 // 256 x 256 4 rows 12.7 (8: 13.8, 16: 17).
+inline long strip_cost(long strips, int H, int layers, int cus, int per_cu, int rows)
+{
+    const long n = strips * ((H + rows - 1) / rows), all = static_cast<long>(per_cu) * cus;
+    return (rows + 3L * (layers + 1)) * (n <= cus ? 3L : (2L + per_cu) * ((n + all - 1) / all));
+}
+
 inline int strip_rows(long strips, int H, int layers, int cus, int per_cu)
 {
     long best = -1;
@@ -136,8 +142,7 @@ inline int strip_rows(long strips, int H, int layers, int cus, int per_cu)
         const long segs = (k ? k * all : cus) / strips;
         if (segs < 1) continue;
         const int r = static_cast<int>(((H + segs - 1) / segs + 1) / 2 * 2);
-        const long n = strips * ((H + r - 1) / r);
-        const long cost = (r + 3L * (layers + 1)) * (n <= cus ? 3L : (2L + per_cu) * ((n + all - 1) / all));
+        const long cost = strip_cost(strips, H, layers, cus, per_cu, r);
         if (best < 0 || cost < best) {
             best = cost;
             rows = r;

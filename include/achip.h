@@ -159,7 +159,8 @@ ACHIP_API int achip_config_info(int precision, int i, int* tw, int* th, int* nt,
 /* Autotuner (project-written; no counterpart in the reference): time every configuration
  * of `precision` on w x h images (src_type -> dst_type) on the net's device, on temporary
  * buffers, a few launches each, and remember the fastest for that size class (log2 of
- * width and height).  Fills *best and, if ms is not NULL, the mean launch time of each
+ * width and height; a 16-bit configuration of a fixed strip height for w x h and the sizes of
+ * the class where that height costs no more than 5% above configuration 0's).  Fills *best and, if ms is not NULL, the mean launch time of each
  * configuration (achip_config_count(precision) floats).  For an FP32 ACNetLegacy net it also
  * times the layer-split form and remembers for achip_pass_ws whether it beat the fastest
  * configuration. */

@@ -157,3 +157,16 @@ def test_strip_height(trace, command, launch, us):
     h = int(command.split()[-1])
     got = [t for r, t in us.items() if -(-h // r) == launches[launch][2]]
     assert got and min(got) <= 1.05 * min(us.values()), launches[launch]
+
+
+def test_tuned_fixed_height_within_its_class(trace):
+    """A tuner's verdict for the 16-bit configuration of 128-row strips (99 against 100 us at 1900 x 1900)
+    holds for that size, and elsewhere in its size class only where 128 rows cost about what the
+    height for the image does; 1100 x 1100 in 128 rows would leave 94 of 256 compute units idle."""
+    tuned, same, other, near = trace(["tune 1 1900 1900 100 99", "legacy 1 -1 1 1900 1900", "legacy 1 -1 1 1100 1100",
+                                      "legacy 1 -1 1 2040 2040"])
+    assert tuned[0] == 1
+    assert same[1][0][1:3] == (30, 15)
+    assert other[1][0][1:3] == (18, 28)   # 40 rows
+    assert near[1][0][1:3] == (32, 16)
+    assert trace(["legacy 1 -1 1 1900 1900"])[0][1][0][2] != 15   # a process that tuned nothing
