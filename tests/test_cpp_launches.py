@@ -170,3 +170,15 @@ def test_tuned_fixed_height_within_its_class(trace):
     assert other[1][0][1:3] == (18, 28)   # 40 rows
     assert near[1][0][1:3] == (32, 16)
     assert trace(["legacy 1 -1 1 1900 1900"])[0][1][0][2] != 15   # a process that tuned nothing
+
+
+@pytest.mark.parametrize("w,h", [(1920, 1080), (640, 360), (256, 256)])
+def test_bench_counts_acnet8_launches(trace, w, h):
+    """The launches from which bench.py derives an ACNet<8> pass's HBM bytes are the ones that run."""
+    import bench
+    precs = ("fp32", "fp16")
+    cases = [(p, b) for p in (0, 1) for b in range(1, 25)]
+    for (p, b), (rc, launches) in zip(cases, trace([f"net8 {b} {p} 1 {w} {h}" for p, b in cases])):
+        assert rc == 0 and len(launches) == bench.acnet8_launches(precs[p], b, w, h), (precs[p], b)
+    assert bench.acnet8_bytes("fp16", 8, 1920, 1080) == 5 * 1920 * 1080
+    assert bench.acnet8_bytes("fp32", 8, 1920, 1080) == (1 + 1 + 4 + 3 * 64) * 1920 * 1080
