@@ -101,7 +101,9 @@ ACHIP_API int achip_pass_batch(ACHipNet* net, int precision, int config, int src
  * net's device, not overlapping src or dst): two launches of four layers on small images, four of
  * two on larger ones (layer 0 with the first), each map through HBM once, a one-pixel recompute
  * ring per layer and launch instead of the fused kernel's eight-pixel halo.  Every output's
- * multiply-adds run in the fused FP32 kernel's order, so the results are its bits.
+ * multiply-adds run in the fused FP32 kernel's order, so for finite sources the results are its
+ * bits.  A NaN or an infinity in an f16 or f32 source gives what the reference's CPU pass gives; the
+ * fused kernel multiplies it by zero weights too and spreads it to neighbours, so there the two differ.
  * The reference's CPU pass runs the layers one by one (CPUProcessor.cpp:1371-1390). */
 ACHIP_API int achip_pass_layers(ACHipNet* net, const void* src, long src_stride, int src_type, int w, int h, void* dst,
                                 long dst_stride, int dst_type, void* workspace, size_t workspace_bytes, void* stream);
@@ -121,7 +123,7 @@ ACHIP_API int achip_pass_batch_layers(ACHipNet* net, int src_type, int dst_type,
  * achip_pass where the caller can lend device memory (the processor's per-thread buffers do;
  * the reference's processors run one form, CUDAProcessor.cpp:383-422).  For FP32 ACNetLegacy
  * passes the forms are the fused kernel and the layer-split form of achip_pass_layers, which
- * give the same bits; the choice is the autotuner's for the size class (achip_autotune times
+ * give the same bits for finite sources; the choice is the autotuner's for the size class (achip_autotune times
  * both), else a rule measured on MI355X: the fused kernel where its 64 x 32 tiles make just about
  * one full round of the device's compute units, the layer-split form elsewhere (1080p u8: 213
  * against 330 us).  achip_pass_ws_bytes gives the

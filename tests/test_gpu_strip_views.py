@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+import oracle_lib as OL
 from anime4kcpp_amd import _native, hip, synth
 
 pytestmark = pytest.mark.gpu
@@ -86,4 +87,27 @@ def test_non_finite_pixels_stay_local(cuda, name, prec, bad):
         inside = np.zeros_like(clean, dtype=bool)
         inside[2 * max(py - rows, 0):2 * (py + rows + 1), 2 * max(px - r, 0):2 * (px + r + 1)] = True
         assert np.array_equal(got[~inside], clean[~inside]), (px, py)
+    net.close()
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("name", ["legacy", "net8", "art f16", "art f32", "fsr f8", "fsr f16"])
+def test_non_finite_pixels_as_the_oracle(cuda, name, bad):
+    """FP32 layers without zero weights: a NaN or an infinity gives the oracle's outputs (max and min take
+    the other operand of a NaN there too)."""
+    w, h = 150, 131
+    x = synth.flat_shaded(7, w, h, dtype=np.float32)
+    x[64, 63] = x[0, 149] = bad
+    s = torch.from_numpy(x).to(cuda)
+    if name == "legacy":
+        net = hip.Net("hdn1")
+        ws = torch.empty(_native.lib().achip_pass8_workspace_bytes(w, h), dtype=torch.uint8, device=cuda)
+        got, want = net.upscale(s, workspace=ws), OL.oracle_pass(x, *hip.load_weights("hdn1"))
+    else:
+        net = NETS[name]()
+        got = net.upscale(s)
+        want = (OL.oracle_pass8(x, *hip.load_weights8("b4_hdn")) if name == "net8" else
+                OL.oracle_artcnn(x, *hip.load_weights_artcnn(name[4:])) if name[:3] == "art" else
+                OL.oracle_fsrcnnx(x, *hip.load_weights_fsrcnnx(name[4:])))
+    assert np.abs(got.cpu().numpy() - want).max() <= 1e-5
     net.close()
