@@ -43,7 +43,11 @@ static Split8 split8(int total, int W, int H, int cus)
     const long strips = (W + (rows8_out<kRowsMap, 2>()) - 1) / (rows8_out<kRowsMap, 2>());
     const bool fours = strips * H <= 12L * (rows8_per_cu<kRowsMap, 2>()) * cus;
     if (total <= 3) return { 1, 0, total - 1 };
-    if (!fours || total == 4) return { total % 2 ? 3 : 2, 0, 2 };
+    // three layers in the head are 512 threads: not for images of more columns than a grid dimension of
+    // 2^32 threads takes that way (487 Mpix; the other launches take any width)
+    const bool wide = (static_cast<long>(W) + rows8_out<kRowsAcnet8, 3>() - 1) / (rows8_out<kRowsAcnet8, 3>()) *
+                          (rows8_threads<kRowsAcnet8, 3>()) >= 1L << 32;
+    if (!fours || total == 4) return { total % 2 ? (wide ? 1 : 3) : 2, 0, 2 };
     switch (total % 4) {
     case 0: return { 4, 0, 4 };
     case 1: return { 3, 1, 4 };

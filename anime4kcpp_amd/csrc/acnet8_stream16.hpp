@@ -60,7 +60,8 @@ struct Chunk8 {
     const uint4* fin;       // 16-bit map in (no image head)
     uint4* fout;            // 16-bit map out (no final layer)
     long ss, ds, fp;
-    int W, H, rows, strips;
+    int W, H, rows;
+    unsigned strips;        // of the image's width
     int l0;                 // block of this launch's layer 1
     int n;                  // layers after layer 0
     unsigned long long roles[2];   // S8Role of every wave, a byte each

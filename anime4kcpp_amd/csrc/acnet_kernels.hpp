@@ -57,7 +57,7 @@ __device__ inline int xcd_tile(int b, int T)
 
 // The grid of strips x segs workgroups of a strip kernel.  A dimension of a grid holds fewer than 2^32
 // threads, so the strips of an image too wide for that (358 Mpix at 768 threads and 64 columns) go along
-// y; strip_block() numbers the workgroups in either form, and a kernel counts its strips from the width.
+// y; strip_block() numbers the workgroups in either form, and a kernel takes its strips from the width.
 inline dim3 strip_grid(long strips, long segs, int threads)
 {
     const unsigned a = static_cast<unsigned>(strips), b = static_cast<unsigned>(segs);

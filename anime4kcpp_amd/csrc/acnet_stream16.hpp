@@ -215,7 +215,8 @@ __global__ __launch_bounds__(kSLThreads, 6) void acnet_stream16(const void* __re
 {
     __shared__ uint4 lds[kSLLds / 16];
     const int t = xcd_tile(strip_block(), gridDim.x * gridDim.y);
-    const int strips = (W + kSLOut - 1) / kSLOut, ty = t / strips, tx = t - ty * strips;
+    const unsigned strips = (static_cast<unsigned>(W) + kSLOut - 1) / kSLOut;
+    const int ty = t / strips, tx = t - ty * strips;
     legacy_strip<T16, TIN, TOUT>(src, ss, W, H, dst, ds, wts, wa, wa0, tx * kSLOut, ty * rows, min((ty + 1) * rows, H),
                                  reinterpret_cast<char*>(lds));
 }

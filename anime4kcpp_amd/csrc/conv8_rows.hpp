@@ -43,7 +43,6 @@ constexpr int kR8In = kR8Cols + 2;                // columns of the first one's 
 constexpr unsigned kR8Row = kR8In * 16;           // bytes of a ring row in one plane (channels 0-3 or 4-7)
 constexpr unsigned kR8Plane = kSRows * kR8Row, kR8Ring = 2 * kR8Plane;
 constexpr unsigned kR8ImgRow = (kR8In + 2) * 4, kR8ImgBytes = kSRows * kR8ImgRow;
-constexpr int kR8Ops = 144 / 16;                  // A-operand registers of an 8 -> 8 layer ([register][lane])
 
 // Output columns of a strip of NL layers after its input or layer 0.
 template <int HEAD, int NL>
@@ -484,7 +483,7 @@ __global__ __launch_bounds__((rows8_threads<HEAD, NL>()), (rows8_waves<HEAD, NL>
     __shared__ float4 lds[rows8_lds<HEAD, NL>() / 16];
     constexpr int out = rows8_out<HEAD, NL>();
     const int t = xcd_tile(strip_block(), gridDim.x * gridDim.y);
-    const int strips = (c.W + out - 1) / out, ty = t / strips, tx = t - ty * strips;
+    const int ty = t / gridDim.x, tx = t - ty * gridDim.x;
     rows8_strip<HEAD, NL, MID, MODE, TIN, TOUT>(c, c.la, c.la[NL - 1], tx * out, out, ty * c.rows,
                                                 min((ty + 1) * c.rows, c.H), (tx + ty) % NL, reinterpret_cast<char*>(lds));
 }
@@ -562,8 +561,8 @@ inline hipError_t launch_rows8(Rows8 c, int cus, hipStream_t stream)
     const int out = rows8_out<HEAD, NL>(), strips = (c.W + out - 1) / out;
     c.rows = rows8_rows(strips, c.H, NL, HEAD == kRowsMap ? 0 : 1, cus, rows8_per_cu<HEAD, NL>());
     constexpr int threads = rows8_threads<HEAD, NL>();
-    hipLaunchKernelGGL((conv8_rows<HEAD, NL, MID, MODE, TIN, TOUT>), strip_grid(strips, (c.H + c.rows - 1) / c.rows, threads),
-                       dim3(threads), 0, stream, c);
+    hipLaunchKernelGGL((conv8_rows<HEAD, NL, MID, MODE, TIN, TOUT>), dim3(strips, (c.H + c.rows - 1) / c.rows), dim3(threads), 0,
+                       stream, c);
     return hipGetLastError();
 }
 

@@ -76,7 +76,7 @@ template <typename TIN, int F, int K>
 __global__ __launch_bounds__(256) void conv_head(const HeadArgs c)
 {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int strips = (c.W + head_cols<F>() - 1) / head_cols<F>(), id = xcd_tile(blockIdx.x, gridDim.x) * 4 + wave;
+    const int strips = (c.W + head_cols<F>() - 1) / head_cols<F>(), id = xcd_tile(strip_block(), gridDim.x * gridDim.y) * 4 + wave;
     const int ty = id / strips, x = (id - ty * strips) * head_cols<F>() + lane / (F / 4), q = lane % (F / 4);
     const int y0 = ty * c.rows, y1 = min(y0 + c.rows, c.H);
     if (y0 >= c.H) return;
@@ -151,7 +151,7 @@ inline hipError_t launch_head(HeadArgs c, int cus, hipStream_t stream)
     const int strips = (c.W + head_cols<F>() - 1) / head_cols<F>();
     c.rows = head_heights(strips, c.H, cus, K == 3 ? 6 : 3, K);
     const int n = strips * ((c.H + c.rows - 1) / c.rows);
-    hipLaunchKernelGGL((conv_head<TIN, F, K>), dim3((n + 3) / 4), dim3(256), 0, stream, c);
+    hipLaunchKernelGGL((conv_head<TIN, F, K>), strip_grid((n + 3) / 4, 1, 256), dim3(256), 0, stream, c);
     return hipGetLastError();
 }
 

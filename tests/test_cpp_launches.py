@@ -73,7 +73,8 @@ def test_acnet8_streamed_lds(trace, blocks):
 
 WIDE = [f"{c} {w} {h}" for w, h in [(360000000, 1), (400000000, 2), (1 << 29, 1)]
         for c in ["net8 8 1 1", "net8 18 2 1", "net8 64 1 1", "net8 4 0 1", "net8 8 0 1", "net8 18 0 516"]]
-WIDE += ["legacy 1 -1 1 360000000 1", "legacy 2 0 516 500000000 1", "layers 1 536870912 1", "batch_layers 3 268435456 1"]
+WIDE += ["legacy 1 -1 1 360000000 1", "legacy 2 0 516 500000000 1", "layers 1 536870912 1", "batch_layers 3 268435456 1",
+         "art 32 4 1 536870912 1"]
 
 
 @pytest.mark.parametrize("command", WIDE)
