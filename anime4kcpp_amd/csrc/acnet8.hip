@@ -43,10 +43,9 @@ static Split8 split8(int total, int W, int H, int cus)
     const long strips = (W + (rows8_out<kRowsMap, 2>()) - 1) / (rows8_out<kRowsMap, 2>());
     const bool fours = strips * H <= 12L * (rows8_per_cu<kRowsMap, 2>()) * cus;
     if (total <= 3) return { 1, 0, total - 1 };
-    // three layers in the head are 512 threads: not for images of more columns than a grid dimension of
-    // 2^32 threads takes that way (487 Mpix; the other launches take any width)
-    const bool wide = (static_cast<long>(W) + rows8_out<kRowsAcnet8, 3>() - 1) / (rows8_out<kRowsAcnet8, 3>()) *
-                          (rows8_threads<kRowsAcnet8, 3>()) >= 1L << 32;
+    // three layers in the head are 512 threads: not for images of more columns than most_strips takes
+    // (487 Mpix; the other launches take any width)
+    const bool wide = (W + rows8_out<kRowsAcnet8, 3>() - 1) / (rows8_out<kRowsAcnet8, 3>()) > most_strips(rows8_threads<kRowsAcnet8, 3>());
     if (!fours || total == 4) return { total % 2 ? (wide ? 1 : 3) : 2, 0, 2 };
     switch (total % 4) {
     case 0: return { 4, 0, 4 };
@@ -205,7 +204,7 @@ static void batch_launch(const SplitDesc* desc, int n, int total, const BatchSpl
     for (int i = 0; i < NL; i++) c.la[i] = legacy_layer(first + i, wts, wa4, nullptr, 0);
     // the first launch writes map 0 (it reads no map), then 0 -> 1 -> 0 -> the outputs
     constexpr int threads = rows8_threads<HEAD, NL>();
-    hipLaunchKernelGGL((conv8_rows_batch<HEAD, NL, kRelu, MODE, TIN, TOUT>), strip_grid(total, 1, threads), dim3(threads), 0, stream, desc, n, total, sp.cols, ((first - 1) / NL & 1) == 0, c);
+    hipLaunchKernelGGL((conv8_rows_batch<HEAD, NL, kRelu, MODE, TIN, TOUT>), strip_row(total, threads), dim3(threads), 0, stream, desc, n, total, sp.cols, ((first - 1) / NL & 1) == 0, c);
 }
 
 template <typename TIN, typename TOUT>

@@ -61,7 +61,7 @@ struct Chunk8 {
     uint4* fout;            // 16-bit map out (no final layer)
     long ss, ds, fp;
     int W, H, rows;
-    unsigned strips;        // of the image's width
+    int tx0;                // first strip of the launch
     int l0;                 // block of this launch's layer 1
     int n;                  // layers after layer 0
     unsigned long long roles[2];   // S8Role of every wave, a byte each
@@ -314,7 +314,8 @@ __global__ __launch_bounds__(64 * kS8MaxWaves, 6) void acnet8_stream16(const Chu
     extern __shared__ uint4 s8_lds[];
     char* const ring0 = reinterpret_cast<char*>(s8_lds) + 16;   // s8_lds_bytes
     char* const img = reinterpret_cast<char*>(s8_lds) + c.n * kSRingBytes + 32;
-    const int t = xcd_tile(strip_block(), gridDim.x * gridDim.y), ty = t / c.strips, tx = t - ty * c.strips;
+    const int t = xcd_tile(strip_block(), gridDim.x * gridDim.y);
+    const int ty = t / gridDim.x, tx = c.tx0 + t - ty * gridDim.x;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const StripRows sr(ty * c.rows, min((ty + 1) * c.rows, c.H), c.H, c.n, IMG ? 1 : 0);
     const int nsteps = sr.steps(), xs = tx * (kSCols - 2 * c.n) - c.n;
@@ -389,15 +390,18 @@ hipError_t s8_launch(Chunk8 c, int cus, hipStream_t stream)
 {
     const int waves = s8_roles(IMG, FINAL, c.n, c.roles);
     if (waves > kS8MaxWaves) return hipErrorInvalidValue;
-    const int out_cols = kSCols - 2 * c.n;
-    c.strips = (c.W + out_cols - 1) / out_cols;
+    const int out_cols = kSCols - 2 * c.n, strips = (c.W + out_cols - 1) / out_cols, most = most_strips(64 * waves);
     const unsigned lds = s8_lds_bytes(IMG, c.n);
     // workgroups per CU: 160 KB of LDS and six waves per SIMD
     const int per_cu = std::min(static_cast<int>(160 * 1024 / lds), 6 / ((waves + 3) / 4));
-    c.rows = strip_rows(c.strips, c.H, c.n, cus, per_cu);
-    hipLaunchKernelGGL((acnet8_stream16<T16, TIN, TOUT, IMG, FINAL>), strip_grid(c.strips, (c.H + c.rows - 1) / c.rows, 64 * waves),
-                       dim3(64 * waves), lds, stream, c);
-    return hipGetLastError();
+    c.rows = strip_rows(strips, c.H, c.n, cus, per_cu);
+    hipError_t e = hipSuccess;
+    for (c.tx0 = 0; c.tx0 < strips && e == hipSuccess; c.tx0 += most) {   // one launch but for very wide images
+        hipLaunchKernelGGL((acnet8_stream16<T16, TIN, TOUT, IMG, FINAL>), dim3(std::min(strips - c.tx0, most), (c.H + c.rows - 1) / c.rows),
+                           dim3(64 * waves), lds, stream, c);
+        e = hipGetLastError();
+    }
+    return e;
 }
 
 template <typename T16, typename TIN, typename TOUT>

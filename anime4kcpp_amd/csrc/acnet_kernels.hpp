@@ -55,14 +55,13 @@ __device__ inline int xcd_tile(int b, int T)
     return x < r ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
 }
 
-// The grid of strips x segs workgroups of a strip kernel.  A dimension of a grid holds fewer than 2^32
-// threads, so the strips of an image too wide for that (358 Mpix at 768 threads and 64 columns) go along
-// y; strip_block() numbers the workgroups in either form, and a kernel takes its strips from the width.
-inline dim3 strip_grid(long strips, long segs, int threads)
-{
-    const unsigned a = static_cast<unsigned>(strips), b = static_cast<unsigned>(segs);
-    return strips * threads < 1L << 32 ? dim3(a, b) : dim3(b, a);
-}
+// A dimension of a grid holds fewer than 2^32 threads.  Strip kernels of an image of more columns than
+// that makes (358 Mpix at 768 threads and 64 columns) go in several launches of most_strips(); those
+// whose workgroups are numbered in one row take the grid's y instead (strip_row).  A kernel finds its
+// strip from gridDim.x either way: a count of its own, from the width or an argument, cost 0.1-0.4 us
+// a launch.
+constexpr int most_strips(int threads) { return static_cast<int>(((1L << 32) - 1) / threads); }
+inline dim3 strip_row(int n, int threads) { return n <= most_strips(threads) ? dim3(n) : dim3(1, n); }
 __device__ inline int strip_block() { return blockIdx.y * gridDim.x + blockIdx.x; }
 
 // Workgroups of a persistent launch: resident workgroups per CU x CUs, at most `tiles`, and

@@ -151,7 +151,7 @@ inline hipError_t launch_head(HeadArgs c, int cus, hipStream_t stream)
     const int strips = (c.W + head_cols<F>() - 1) / head_cols<F>();
     c.rows = head_heights(strips, c.H, cus, K == 3 ? 6 : 3, K);
     const int n = strips * ((c.H + c.rows - 1) / c.rows);
-    hipLaunchKernelGGL((conv_head<TIN, F, K>), strip_grid((n + 3) / 4, 1, 256), dim3(256), 0, stream, c);
+    hipLaunchKernelGGL((conv_head<TIN, F, K>), strip_row((n + 3) / 4, 256), dim3(256), 0, stream, c);
     return hipGetLastError();
 }
 
