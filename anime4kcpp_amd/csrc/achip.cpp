@@ -255,8 +255,8 @@ std::map<std::tuple<int, int, int, int, int, int>, bool> g_split;
 
 // The form achip_pass_ws runs: the layer-split one only for FP32 ACNetLegacy passes, and there
 // the autotuner's verdict for the size class, else this rule: the fused kernel, which needs no
-// workspace, where its 64 x 32 tiles make just about one full round of the compute units (within 4%
-// of the split form there), the split form elsewhere.  u8, fused / split us: 128 x 96 81 / 20,
+// workspace of 64 bytes per pixel, where its 64 x 32 tiles make just about one full round of the
+// compute units (the split form gains at most 4% there), the split form elsewhere.  u8, fused / split us: 128 x 96 81 / 20,
 // 256 x 256 83 / 28, 720 x 480 84 / 61, 960 x 540 84 / 81 (one tile per compute unit), 1280 x 720
 // 165 / 118, 1920 x 1080 330 / 213, 3840 x 2160 1310 / 780.
 bool split_preferred(const ACHipNet* net, int precision, int st, int dt, int w, int h)

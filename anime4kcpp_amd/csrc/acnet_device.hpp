@@ -42,8 +42,8 @@ constexpr int kMfma32BlobFloats = kMfma32L0Floats + 8 * kMfma32LayerFloats;   //
 // ACNet<8> device blob (model arrays of core/include/AC/Core/Model/ACNet.hpp:63-118,
 // repacked): L0 weights w0[p][n] (72), bias (8), PReLU slopes (8); the final layer's 4
 // biases (padded to 8); then per block l = 1..B its 8 biases and 8 slopes.  The conv weights
-// of the blocks and of the final 8 -> 4 layer (output channels 4-7 zero) are FP32 MFMA
-// per-lane A operands, kMfma32LayerFloats per layer (layout of the legacy layers 1..8).
+// of the blocks and of the final 8 -> 4 layer are 4x4x1 MFMA operands, kRows8Floats per layer
+// (acnet_kernels.hpp; pack_conv8_operands), and the 16-bit ones 3 x 64 x 8 values per layer.
 constexpr int kA8OffW0 = 0, kA8OffB0 = 72, kA8OffAlpha0 = 80, kA8OffFinalB = 88, kA8OffLayer = 96;
 __host__ __device__ constexpr int acnet8_blob_floats(int blocks) { return kA8OffLayer + 16 * blocks; }
 

@@ -118,20 +118,21 @@ __device__ __forceinline__ void strip_loader(const void* __restrict__ src, long 
 // the lag of the layers and the loader.
 inline int strip_steps(int rows, int layers) { return (rows + 1) / 2 + kSLag * (layers + 1); }
 
-// Rows per strip of an image of `strips` strips x H rows on a device of `cus` compute units that
-// hold per_cu workgroups each.  Measured (u8 in FP16, 4 to 18 blocks and ACNetLegacy, 256 x 256 to 4K): a
-// strip of r rows with a compute unit of its own takes time with r + 3 (layers + 1) (the steps that
-// fill and drain it, two per layer, run fewer layers than the rest), two to a compute unit 4/3 of that.
-// So the candidates are the heights that fill one workgroup per CU or 1, 2, 4 rounds of all, and the
-// cheapest by that count is taken.  ACNetLegacy, us: 1080p 64 rows 47 (36: 58, 80: 55); 4K 270 rows 150
-// (128: 149, 64: 163); 800 x 600 16 rows 21.8 (32 rows, one per CU: 23.7; 64 x 32 tiles before: 23.1);
-// 256 x 256 4 rows 12.7 (8: 13.8, 16: 17).
+// What strips of `rows` rows of an image of `strips` strips x H rows take on a device of `cus` compute
+// units that hold per_cu workgroups each.  Measured (u8 in FP16, 4 to 18 blocks and ACNetLegacy,
+// 256 x 256 to 4K): a strip of r rows with a compute unit of its own takes time with r + 3 (layers + 1)
+// (the steps that fill and drain it, two per layer, run fewer layers than the rest), two to a compute
+// unit 4/3 of that.
 inline long strip_cost(long strips, int H, int layers, int cus, int per_cu, int rows)
 {
     const long n = strips * ((H + rows - 1) / rows), all = static_cast<long>(per_cu) * cus;
     return (rows + 3L * (layers + 1)) * (n <= cus ? 3L : (2L + per_cu) * ((n + all - 1) / all));
 }
 
+// Rows per strip: the heights that fill one workgroup per CU or 1, 2, 4 rounds of all, the cheapest by
+// that count.  ACNetLegacy, us: 1080p 64 rows 47 (36: 58, 80: 55); 4K 270 rows 150 (128: 149, 64: 163);
+// 800 x 600 16 rows 21.8 (32 rows, one per CU: 23.7; 64 x 32 tiles before: 22); 256 x 256 4 rows 12.7
+// (8: 13.8, 16: 17).
 inline int strip_rows(long strips, int H, int layers, int cus, int per_cu)
 {
     long best = -1;
